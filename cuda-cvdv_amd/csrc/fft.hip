@@ -29,6 +29,7 @@
 #include "cvdv_internal.h"
 #include "diag_fast.h"
 #include "fft_bfly.h"
+#include "fft_stages.h"
 
 static const long double PI_L = 3.141592653589793238462643383279502884L;
 
@@ -314,69 +315,6 @@ __device__ __forceinline__ double2 lane_value(double2 v, int lane) {
     return make_double2(rd(v.x), rd(v.y));
 }
 
-// LDS layouts of the Stockham exchanges (padding breaks power-of-two strides).
-// LAY 0, every exchange of every tile unless below: one pad entry per 32.
-// One-row complex64 tiles of 2^13-2^14 points write exchange 0 at a stride of 8
-// entries and exchange 1 in runs of 8 lanes 64 entries apart, which puts two
-// lanes of every 16 on one LDS bank under LAY 0: there exchange 0 takes one pad
-// entry per 16 (LAY 1) and exchange 1 eight per 64 (LAY 2).
-template <int LAY>
-__device__ __forceinline__ int lay_ix(int i) {
-    return LAY == 0 ? i + (i >> 5) : (LAY == 1 ? i + (i >> 4) : i + ((i >> 6) << 3));
-}
-template <int LAY> constexpr int lay_period() { return LAY == 0 ? 32 : (LAY == 1 ? 16 : 64); }
-template <int LAY> constexpr int lay_padded(int stride) {
-    return stride + (LAY == 0 ? stride / 32 : (LAY == 1 ? stride / 16 : stride / 8));
-}
-// The layout of exchange XS (stage XS's outputs, read by stage XS + 1).
-template <bool ONE, int XS> constexpr int ex_lay() { return !ONE ? 0 : (XS == 0 ? 1 : (XS == 1 ? 2 : 0)); }
-
-__device__ __forceinline__ int lds_ix(int i) { return lay_ix<0>(i); }
-
-// Padded index of i0 + m * STRIDE.  When STRIDE is a multiple of the layout's
-// period the padding is linear (adding it leaves the bits below the period
-// alone), so every element is the padded base plus a compile-time offset (an
-// immediate in the LDS access).
-template <int STRIDE, int LAY = 0>
-__device__ __forceinline__ int lds_at(int i0, int pbase, int m) {
-    if constexpr (STRIDE % lay_period<LAY>() == 0) return pbase + m * lay_padded<LAY>(STRIDE);
-    else return lay_ix<LAY>(i0 + m * STRIDE);
-}
-
-// Stage plan of a length-2^LGM transform: radix-8 stages, then one radix-4 or
-// radix-2 stage.  Stage s has sub-length L = 8^s and its twiddles start at
-// entry off(s) of the stage table (W_{RL}^{ij} at off + j (R-1) + i - 1), the
-// layout stage_values() writes.
-template <int LGM> struct Plan {
-    static constexpr int NST = LGM / 3 + (LGM % 3 ? 1 : 0);
-    static constexpr int lgr(int s) { return s < LGM / 3 ? 3 : LGM % 3; }
-    static constexpr int off(int s) {
-        int o = 0, L = 1;
-        for (int i = 0; i < s; ++i) {
-            o += L * ((1 << lgr(i)) - 1);
-            L <<= lgr(i);
-        }
-        return o;
-    }
-};
-
-// Offsets of the split twiddle table (split_values) for stage s of a length-2^LGM
-// transform: the direct segment (L <= 64) or the a and b segments.
-template <int LGM> struct SplitPlan {
-    static constexpr int seg(int s) {  // entries of stage s
-        const int R = 1 << Plan<LGM>::lgr(s), L = 1 << (3 * s);
-        return s == 0 ? 0 : (L <= 64 ? L * (R - 1) : (L / 64) * (R - 1) + 64 * (R - 1));
-    }
-    static constexpr int off(int s) {
-        int o = 0;
-        for (int i = 0; i < s; ++i) o += seg(i);
-        return o;
-    }
-    static constexpr int total() { return off(Plan<LGM>::NST); }
-};
-
-// ---------------------------------------------------------------- butterflies (fft_bfly.h)
-
 // Tile element e (linear) -> (c, row, hb) in the given order.
 template <int LGM>
 __device__ __forceinline__ void tile_coords(int e, int lgC, int lgHb, int rowFast, int& c, int& row, int& hb) {
@@ -386,105 +324,6 @@ __device__ __forceinline__ void tile_coords(int e, int lgC, int lgHb, int rowFas
     const int lo = rest & ((1 << lgLo) - 1), hi = rest >> lgLo;
     row = rowFast ? lo : hi;
     hb = rowFast ? hi : lo;
-}
-
-// Stockham stage geometry.  Butterfly b of a stage of radix RP (sub-length
-// L = 2^lgL already transformed) takes rows q + i*M/RP of column c in block hb
-// and writes rows ob + m*L, ob = hb*M + (q/L)*RP*L + (q mod L); every thread
-// owns E/RP butterflies b = tid + k*nt.
-struct BflyPos {
-    int c, q, hb;
-};
-
-template <int RP, int LGM>
-__device__ __forceinline__ BflyPos bfly_pos(int b, int lgC) {
-    constexpr int LGR = RP == 8 ? 3 : (RP == 4 ? 2 : 1);
-    constexpr int lgMq = LGM - LGR;
-    BflyPos p;
-    p.c = b & ((1 << lgC) - 1);
-    const int rest = b >> lgC;
-    p.q = rest & ((1 << lgMq) - 1);
-    p.hb = rest >> lgMq;
-    return p;
-}
-
-// Twiddle the inputs of the butterflies in x (stage S, radix RP) and transform.
-// TWL: the twiddles are the split table staged in LDS (one-row tiles), else the
-// stage table in global memory.
-template <int RP, int E, int LGM, int LGC, int S, bool TWL, typename C>
-__device__ __forceinline__ void stage_compute(C* x, const C* __restrict__ tw, int tid, int nt) {
-    constexpr int lgC = LGC;
-    constexpr int NB = E / RP;
-    constexpr int lgL = 3 * S;
-#pragma unroll
-    for (int k = 0; k < NB; ++k) {
-        if (lgL > 0) {
-            const BflyPos p = bfly_pos<RP, LGM>(tid + k * nt, lgC);
-            const int pq = p.q & ((1 << lgL) - 1);
-            if constexpr (!TWL) {
-                const C* t = tw + Plan<LGM>::off(S) + pq * (RP - 1);
-#pragma unroll
-                for (int i = 1; i < RP; ++i) x[k * RP + i] = cmul(x[k * RP + i], t[i - 1]);
-            } else if constexpr (lgL <= 6) {
-                const C* t = tw + SplitPlan<LGM>::off(S) + pq;
-#pragma unroll
-                for (int i = 1; i < RP; ++i) x[k * RP + i] = cmul(x[k * RP + i], t[(i - 1) << lgL]);
-            } else {
-                constexpr int LA = (1 << lgL) / 64;
-                constexpr int OA = SplitPlan<LGM>::off(S);
-                constexpr int OB = OA + LA * (RP - 1);
-                const C* ta = tw + OA + (pq >> 6);
-                const C* tb = tw + OB + (pq & 63);
-#pragma unroll
-                for (int i = 1; i < RP; ++i)
-                    x[k * RP + i] = cmul(x[k * RP + i], cmul(ta[(i - 1) * LA], tb[(i - 1) * 64]));
-            }
-        }
-        dft_r<RP, false>(x + k * RP);
-    }
-}
-
-// Outputs of stage S (radix RP) -> LDS in Stockham order (exchange S; ONE: the
-// one-row layouts).
-template <int RP, int E, int LGM, int LGC, int S, bool ONE = false, typename C>
-__device__ __forceinline__ void stage_write(C* lds, const C* x, int tid, int nt) {
-    constexpr int LAY = ex_lay<ONE, S>();
-    constexpr int NB = E / RP;
-    constexpr int LGR = RP == 8 ? 3 : (RP == 4 ? 2 : 1);
-    constexpr int lgL = 3 * S;
-    constexpr int STRIDE = 1 << (lgL + LGC);
-#pragma unroll
-    for (int k = 0; k < NB; ++k) {
-        const BflyPos p = bfly_pos<RP, LGM>(tid + k * nt, LGC);
-        const int ob = (p.hb << LGM) + ((p.q >> lgL) << (LGR + lgL)) + (p.q & ((1 << lgL) - 1));
-        const int i0 = (ob << LGC) + p.c, pb = lay_ix<LAY>(i0);
-        if constexpr (LAY != 0) {
-            // one-row exchanges 0 and 1: i0 = 8q with entries i0 + m (period 16),
-            // or i0 mod 64 < 8 with entries i0 + 8m (period 64): all within i0's period
-#pragma unroll
-            for (int m = 0; m < RP; ++m) lds[pb + m * STRIDE] = x[k * RP + m];
-        } else {
-#pragma unroll
-            for (int m = 0; m < RP; ++m) lds[lds_at<STRIDE, LAY>(i0, pb, m)] = x[k * RP + m];
-        }
-    }
-}
-
-// Inputs of a stage of radix RP <- LDS (exchange XS).
-template <int RP, int E, int LGM, int LGC, int XS = 0, bool ONE = false, typename C>
-__device__ __forceinline__ void stage_read(const C* lds, C* x, int tid, int nt) {
-    constexpr int LAY = ex_lay<ONE, XS>();
-    constexpr int NB = E / RP;
-    constexpr int LGR = RP == 8 ? 3 : (RP == 4 ? 2 : 1);
-    constexpr int lgMq = LGM - LGR;
-    constexpr int STRIDE = 1 << (lgMq + LGC);
-#pragma unroll
-    for (int k = 0; k < NB; ++k) {
-        const BflyPos p = bfly_pos<RP, LGM>(tid + k * nt, LGC);
-        const int i0 = (((p.hb << LGM) + p.q) << LGC) + p.c, pb = lay_ix<LAY>(i0);
-#pragma unroll
-        for (int i = 0; i < RP; ++i) x[k * RP + i] = lds[lds_at<STRIDE, LAY>(i0, pb, i)];
-    }
 }
 
 // The compiled pending program, staged in LDS so its runtime-length loops read
@@ -918,22 +757,6 @@ __device__ __forceinline__ void last_store(C* __restrict__ out, const C* v, cons
     }
 }
 
-// Stages 1 .. NST-1: exchange the previous stage's outputs through LDS, then
-// twiddle and transform.
-template <int LGM, int LGC, int S, int E, bool TWL, bool ONE = false, typename C>
-__device__ __forceinline__ void run_stages(C* x, C* lds, const C* __restrict__ tw, int tid, int nt) {
-    if constexpr (S < Plan<LGM>::NST) {
-        constexpr int RPprev = 1 << Plan<LGM>::lgr(S - 1);
-        constexpr int RP = 1 << Plan<LGM>::lgr(S);
-        stage_write<RPprev, E, LGM, LGC, S - 1, ONE>(lds, x, tid, nt);
-        lds_barrier();
-        stage_read<RP, E, LGM, LGC, S - 1, ONE>(lds, x, tid, nt);
-        lds_barrier();
-        stage_compute<RP, E, LGM, LGC, S, TWL>(x, tw, tid, nt);
-        run_stages<LGM, LGC, S + 1, E, TWL, ONE>(x, lds, tw, tid, nt);
-    }
-}
-
 // One-row complex64 tiles of 2^13-2^14 points lay out their first two exchanges
 // apart from the others (ex_lay); their LDS ends at tile + tile/8.
 template <typename R, int LGM, int LGC>
@@ -1024,7 +847,7 @@ k_fft_tile(const typename CT<R>::type* in, typename CT<R>::type* out, FftPass d,
     // Transform the phased tile in registers (the last stage's outputs stay in x).
     auto stages = [&](C* x, int ti, const C* twt) {
         stage_compute<R0, E, LGM, LGC, 0, PF>(x, twt, ti, nt);
-        run_stages<LGM, LGC, 1, E, PF, ONE>(x, lds, twt, ti, nt);
+        run_stages<LGM, LGC, 1, E, PF, ONE ? EX_ONE : EX_TILE>(x, lds, twt, ti, nt);
     };
     // Store the transformed tile t.
     // Staged store, first half: the last stage's outputs into LDS in natural order.
