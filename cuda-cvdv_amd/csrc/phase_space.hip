@@ -16,11 +16,10 @@
 
 #include <cmath>
 #include <string>
-#include <type_traits>
 #include <vector>
 
 #include "cvdv_internal.h"
-#include "fft_stages.h"
+#include "readout_rows.h"
 #include "../../include/cvdv_hip.h"
 
 static const double PI = 3.14159265358979323846;
@@ -187,17 +186,7 @@ __global__ void k_real_clamp(double* __restrict__ out, const double2* __restrict
 // ---------------------------------------------------------------- row kernels
 // Native grids of 2^3 .. 2^13 points: one workgroup builds its rows' integrands in
 // registers, transforms them in LDS (fft_stages.h) and writes the picture, so no
-// N x N intermediate touches memory.  A tile is Hb rows of N points, eight points a
-// thread: whole rows from 2^9 points on, 512 points of several rows below.
-#define ROWS_LGM_MIN 3
-#define ROWS_LGM_MAX 13
-template <int LGM> constexpr int rows_lg_hb() { return LGM >= 9 ? 0 : 9 - LGM; }
-template <int LGM> constexpr int rows_threads() { return 1 << (LGM + rows_lg_hb<LGM>() - 3); }
-template <int LGM> constexpr size_t rows_lds() {
-    constexpr int tile = 1 << (LGM + rows_lg_hb<LGM>());
-    return (size_t)(tile + tile / 8) * sizeof(double2);  // EX_ROWS layout
-}
-
+// N x N intermediate touches memory.
 // Slice s of a contiguous register field, point j (logical), widened to FP64.
 template <typename C>
 __device__ __forceinline__ double2 slice_at(const C* __restrict__ X, uint64_t s, int lgN, int j, int refl) {
@@ -452,20 +441,6 @@ static Bufs extract_slices(CVDVContext* ctx, int r, double2* X) {
     return b;
 }
 
-// Calls f with the register's size as a compile-time constant (ROWS_LGM_MIN ..
-// ROWS_LGM_MAX points).
-template <typename F>
-static void rows_dispatch(int n, F f) {
-    switch (n) {
-#define CVDV_ROWS_CASE(L) \
-    case L: f(std::integral_constant<int, L>{}); break;
-        CVDV_ROWS_CASE(3) CVDV_ROWS_CASE(4) CVDV_ROWS_CASE(5) CVDV_ROWS_CASE(6) CVDV_ROWS_CASE(7) CVDV_ROWS_CASE(8)
-        CVDV_ROWS_CASE(9) CVDV_ROWS_CASE(10) CVDV_ROWS_CASE(11) CVDV_ROWS_CASE(12) CVDV_ROWS_CASE(13)
-#undef CVDV_ROWS_CASE
-        default: throw CvdvError{CVDV_ERR_UNSUPPORTED, "readout row length without a kernel instance"};
-    }
-}
-
 // The rows kernels read the slices of a contiguous field from the state itself, those
 // of any other field from the extracted copy X.
 struct RowsIn {
@@ -480,12 +455,6 @@ static RowsIn rows_input(CVDVContext* ctx, int r, double2* X) {
     if (rows_direct(ctx, r)) return RowsIn{ctx->state(), ctx->prec == CVDV_C128, ctx->refl[r]};
     extract_slices(ctx, r, X);
     return RowsIn{X, true, 0};
-}
-
-template <typename K>
-static void rows_launch_attr(K kfn, size_t lds) {
-    if (lds > 64 * 1024)
-        HIPCHK(hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
 }
 
 // Every pair of rows reads the slices again, where k_rho's tiles share them: with many
