@@ -224,6 +224,25 @@ struct FtDefers {
     }
 };
 
+// Transforms of one register field collected while a gate runs, launched together by
+// chain_flush (fft_chain.hip).  Anything else that touches the state launches them
+// first, and a gate never returns with any left.
+#define FT_CHAIN_MAX 4      // transforms of one launch (a squeezing gate's)
+#define FT_CHAIN_TERMS 6    // phase terms of one transform
+#define FT_CHAIN_LG_SMALL 22  // states up to 2^22: every transform of a fitting field
+#define FT_CHAIN_LG_MAX 30    // largest state (32-bit element indices)
+struct FtChainStep {
+    DiagProg prog;
+    int inverse;
+    double scale;
+};
+struct FtChain {
+    int open = 0;  // a gate is collecting
+    int n = 0;
+    int sh = 0, nb = 0;
+    FtChainStep st[FT_CHAIN_MAX];
+};
+
 // Host-side state at the start of a graph capture (restored at its end: nothing
 // has executed).  Kept per context, so captures on several contexts may nest.
 struct CaptureSave {
@@ -248,6 +267,7 @@ struct CVDVContext {
     hipStream_t stream = nullptr;
     DiagProg pending{};
     FtDefers defer{};                 // half-done register transforms (fft.hip)
+    FtChain chain;                    // transforms the current gate has collected (fft_chain.hip)
     int fuseFt = 1;                   // 0: every transform runs whole (no deferred halves)
     std::map<uint64_t, FftCfg> fftCfg;  // tuned tile choices per register field (fft_cfg_key)
     size_t freeMemOverride = 0;       // readout route choice: assumed free device bytes (0 = ask)
@@ -319,6 +339,15 @@ CVDVContext* ctx_create_like(const CVDVContext* src);
 void fft_settle_for(CVDVContext* ctx, const DiagProg& p, uint64_t except = 0);
 // Complete a half-done transform when the bits `mask` overlap its field.
 void fft_settle_bits(CVDVContext* ctx, uint64_t mask);
+
+// fft_chain.hip
+// A transform of field [sh, sh+nb) joins the current gate's chain (launched at once
+// outside a gate); false when it has to run by itself, nothing done.
+bool chain_accept(CVDVContext* ctx, int sh, int nb, bool inverse, const DiagProg& pre, double outScale);
+bool chain_field(const CVDVContext* ctx, int sh, int nb);  // its transforms run as chains
+void chain_flush(CVDVContext* ctx);                        // launch what was collected
+// fft.hip: a transform by itself (halves kept pending, or whole)
+void fft_whole(CVDVContext* ctx, int sh, int nb, bool inverse, const DiagProg& pre, double outScale);
 
 // measure.hip
 void marginal_probs(CVDVContext* ctx, const int* regs, int nsel, double* hostOut);

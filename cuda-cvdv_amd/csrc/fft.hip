@@ -1587,6 +1587,7 @@ static void settle_impl(CVDVContext* ctx, const FtDefer D) {
 }
 
 static void settle_one(CVDVContext* ctx, FtDefer& rec) {
+    chain_flush(ctx);
     const FtDefer D = rec;
     rec = FtDefer{};
     if (ctx->prec == CVDV_C128) settle_impl<double>(ctx, D);
@@ -1712,17 +1713,26 @@ void fft_prepare(CVDVContext* ctx) {
 
 void fft_register(CVDVContext* ctx, int pshift, int nbits, bool inverse, const DiagProg& pre,
                   double outScale) {
-    const bool done = ctx->prec == CVDV_C128 ? fft_deferred<double>(ctx, pshift, nbits, inverse, pre, outScale)
-                                             : fft_deferred<float>(ctx, pshift, nbits, inverse, pre, outScale);
+    if (chain_field(ctx, pshift, nbits)) {
+        if (FtDefer* rec = ctx->defer.find(pshift)) settle_one(ctx, *rec);
+        if (chain_accept(ctx, pshift, nbits, inverse, pre, outScale)) return;
+    }
+    chain_flush(ctx);
+    fft_whole(ctx, pshift, nbits, inverse, pre, outScale);
+}
+
+void fft_whole(CVDVContext* ctx, int sh, int nb, bool inverse, const DiagProg& pre, double outScale) {
+    const bool done = ctx->prec == CVDV_C128 ? fft_deferred<double>(ctx, sh, nb, inverse, pre, outScale)
+                                             : fft_deferred<float>(ctx, sh, nb, inverse, pre, outScale);
     if (done) return;
-    if (FtDefer* rec = ctx->defer.find(pshift)) settle_one(ctx, *rec);
+    if (FtDefer* rec = ctx->defer.find(sh)) settle_one(ctx, *rec);
     bool swapped;
     if (ctx->prec == CVDV_C128)
         swapped = fft_run<double>(ctx, (double2*)ctx->state(), [ctx] { return (double2*)ctx->other(); },
-                                  ctx->totalSize, pshift, nbits, inverse, pre, outScale, CVDV_C128);
+                                  ctx->totalSize, sh, nb, inverse, pre, outScale, CVDV_C128);
     else
         swapped = fft_run<float>(ctx, (float2*)ctx->state(), [ctx] { return (float2*)ctx->other(); },
-                                 ctx->totalSize, pshift, nbits, inverse, pre, outScale, CVDV_MIXED);
+                                 ctx->totalSize, sh, nb, inverse, pre, outScale, CVDV_MIXED);
     if (swapped) ctx->cur = 1 - ctx->cur;
 }
 

@@ -219,6 +219,7 @@ static bool term_is_identity(const DiagTerm& t) {
 // The whole program as one FP64 pass over the state (programs that exceed the
 // compiled capacities).
 static void diag_prog_pass(CVDVContext* ctx, const DiagProg& p) {
+    chain_flush(ctx);
     fft_settle_for(ctx, p);
     const uint64_t n = ctx->totalSize;
     const int pid = prof_begin(ctx, KK_DIAG);
@@ -567,6 +568,7 @@ void launch_diag(CVDVContext* ctx, const DiagProg& pp) {
         rec_op(ctx, op, pp);
         return;
     }
+    chain_flush(ctx);
     fft_settle_for(ctx, pp);
     const uint64_t n = ctx->totalSize;
     bool act;
@@ -732,6 +734,7 @@ static void qubit_gate(CVDVContext* ctx, int reg, int qubit, const double m[8]) 
         rec_op(ctx, op, ctx_take_involving(ctx, 1ull << bit));
         return;
     }
+    chain_flush(ctx);
     fft_settle_bits(ctx, 1ull << bit);
     const DiagProg taken = ctx_take_involving(ctx, 1ull << bit);
     fft_settle_for(ctx, taken);
@@ -802,6 +805,7 @@ static void cparity(CVDVContext* ctx, int tgt, int creg, int cq) {
         rec_op(ctx, op, ctx_take_involving(ctx, (((uint64_t)1 << nb) - 1ull) << ctx->pshift[tgt]));
         return;
     }
+    chain_flush(ctx);
     fft_settle_bits(ctx, ((((uint64_t)1 << nb) - 1ull) << ctx->pshift[tgt]) | (1ull << cpos));
     const DiagProg taken = ctx_take_involving(ctx, (((uint64_t)1 << nb) - 1ull) << ctx->pshift[tgt]);
     fft_settle_for(ctx, taken);
@@ -837,8 +841,28 @@ static void phase_bilin(CVDVContext* ctx, int r1, int r2, double c, int creg = -
 }
 
 // ---------------------------------------------------------------- validation
-#define CVDV_TRY try {
+// A gate's transforms of one field are launched together (FtChain): collected while
+// the scope is open, launched when it closes, also when the gate fails half way.
+struct ChainScope {
+    CVDVContext* ctx;
+    explicit ChainScope(CVDVContext* c) : ctx(c) { ctx->chain.open = 1; }
+    void close() {
+        ctx->chain.open = 0;
+        chain_flush(ctx);
+    }
+    ~ChainScope() {
+        ctx->chain.open = 0;
+        if (ctx->chain.n == 0) return;
+        try {
+            chain_flush(ctx);
+        } catch (...) {
+        }
+    }
+};
+
+#define CVDV_TRY try { ChainScope scope(ctx);
 #define CVDV_CATCH()                                                         \
+        scope.close();                                                       \
     }                                                                        \
     catch (const CvdvError& e) {                                             \
         cvdv_set_error(e.code, e.msg);                                       \
@@ -924,15 +948,19 @@ static void bs_small(CVDVContext* ctx, int r1, int r2, double th, int c = -1, in
     // phases read its bits).  Otherwise the register with the lower physical
     // field goes first, since its rows are contiguous, where the phase reduces to
     // one affine term per row instead of a per-element evaluation.
-    const bool d1 = fft_defers(ctx, ctx->pshift[r1], ctx->nq[r1]);
-    const bool d2 = fft_defers(ctx, ctx->pshift[r2], ctx->nq[r2]);
+    auto chains = [ctx](int r) { return !ctx->rec && chain_field(ctx, ctx->pshift[r], ctx->nq[r]); };
+    const bool d1 = !chains(r1) && fft_defers(ctx, ctx->pshift[r1], ctx->nq[r1]);
+    const bool d2 = !chains(r2) && fft_defers(ctx, ctx->pshift[r2], ctx->nq[r2]);
     int fa = ctx->pshift[r1] <= ctx->pshift[r2] ? r1 : r2;
     if (d1 != d2) fa = d1 ? r1 : r2;
-    const int fb = fa == r1 ? r2 : r1;
+    int fb = fa == r1 ? r2 : r1;
     phase_bilin(ctx, r1, r2, cq, c, q);
     ctx_ft(ctx, fa, false);
     ctx_ft(ctx, fb, false);
     phase_bilin(ctx, r1, r2, cp, c, q);
+    // where transforms run as chains, the second register's pair and the phase between
+    // take one launch
+    if (chains(fb) && !(d1 || d2)) std::swap(fa, fb);
     ctx_ft(ctx, fa, true);
     ctx_ft(ctx, fb, true);
     phase_bilin(ctx, r1, r2, cq, c, q);
