@@ -179,7 +179,7 @@ struct ProfRec {
 };
 
 // A register transform left half done (fft.hip).  The four-step FFT of a
-// register field of 2n bits (digits lo = bits [sh, sh+n), hi = [sh+n, sh+2n))
+// register field of n1 + n2 bits (digits lo = bits [sh, sh+n1), hi the n2 above them)
 // is two in-place half passes: H (transform over hi) and L (twiddle W_N^{lo*hi},
 // transform over lo).  After H the second half is pending (!high: L, whose
 // in-place result is the momentum register with its digits exchanged); after L

@@ -400,7 +400,7 @@ __device__ __forceinline__ void stage0_load(const C* __restrict__ in, C* x, cons
     constexpr int lgMq = LGM - LGR;
 #pragma unroll
     for (int k = 0; k < NB; ++k) {
-        const BflyPos p = bfly_pos<RP, LGM>(tid + k * nt, LGC);
+        const BflyPos p = bfly_pos<RP, LGM, E>(tid, k, nt, LGC);
         const uint64_t g0 = inBase + ((uint64_t)p.hb << d.lgInH2) + ((uint64_t)p.q << d.lgInR) + p.c;
 #pragma unroll
         for (int i = 0; i < RP; ++i) x[k * RP + i] = in[g0 + ((uint64_t)(i << lgMq) << d.lgInR)];
@@ -443,7 +443,7 @@ __device__ __forceinline__ void stage0_pre(C* x, const FftPass& d, uint64_t inBa
             for (int i = 1; i < RP; ++i) st[i] = tw4[(k2 * (uint32_t)(i << lgMq)) & nmask];
 #pragma unroll
             for (int k = 0; k < NB; ++k) {
-                const BflyPos p = bfly_pos<RP, LGM>(tid + k * nt, LGC);
+                const BflyPos p = bfly_pos<RP, LGM, E>(tid, k, nt, LGC);
                 const C b = tw4[(k2 * (uint32_t)p.q) & nmask];
                 x[k * RP] = cmul(x[k * RP], b);
 #pragma unroll
@@ -456,7 +456,7 @@ __device__ __forceinline__ void stage0_pre(C* x, const FftPass& d, uint64_t inBa
             // depth log2(RP)
 #pragma unroll
             for (int k = 0; k < NB; ++k) {
-                const BflyPos p = bfly_pos<RP, LGM>(tid + k * nt, LGC);
+                const BflyPos p = bfly_pos<RP, LGM, E>(tid, k, nt, LGC);
                 const uint64_t g0 = inBase + ((uint64_t)p.hb << d.lgInH2) + ((uint64_t)p.q << d.lgInR) + p.c;
                 const uint32_t nmask = (1u << d.tw4LogN) - 1u;
                 const uint32_t k2 = (uint32_t)(g0 >> d.tw4Shift) & ((1u << d.tw4HiBits) - 1u);
@@ -474,7 +474,7 @@ __device__ __forceinline__ void stage0_pre(C* x, const FftPass& d, uint64_t inBa
     if (TM != TM_NONE && d.usePre) {
         int tt = tid;
         auto elem = [&](int k, int i) {
-            const BflyPos p = bfly_pos<RP, LGM>(tt + k * nt, LGC);
+            const BflyPos p = bfly_pos<RP, LGM, E>(tt, k, nt, LGC);
             return inBase + ((uint64_t)p.hb << d.lgInH2) + ((uint64_t)p.q << d.lgInR) + p.c +
                    ((uint64_t)(i << lgMq) << d.lgInR);
         };
@@ -540,7 +540,7 @@ __device__ __forceinline__ void stage0_pre(C* x, const FftPass& d, uint64_t inBa
                     C e[CH];
 #pragma unroll
                     for (int j = 0; j < CH; ++j) {
-                        const BflyPos p = bfly_pos<RP, LGM>(tt + ((j0 + j) / RP) * nt, LGC);
+                        const BflyPos p = bfly_pos<RP, LGM, E>(tt, (j0 + j) / RP, nt, LGC);
                         const uint32_t row = (uint32_t)(p.q + (((j0 + j) % RP) << lgMq));
                         e[j] = tb[s < 31 ? (row << s) : 0u];
                         if (cj) e[j].y = -e[j].y;
@@ -590,7 +590,7 @@ __device__ __forceinline__ void stage0_pre(C* x, const FftPass& d, uint64_t inBa
             lds_barrier();
 #pragma unroll
             for (int k = 0; k < NB; ++k) {
-                const BflyPos p = bfly_pos<RP, LGM>(tt + k * nt, LGC);
+                const BflyPos p = bfly_pos<RP, LGM, E>(tt, k, nt, LGC);
                 const uint64_t g0 = elem(k, 0);
                 double p0 = pre.genrev;
                 for (int t = 0; t < pre.ngen; ++t) p0 += cvdv_frac(diag_term_rev(P.gen[t], g0));
@@ -625,7 +625,7 @@ __device__ __forceinline__ void stage0_pre(C* x, const FftPass& d, uint64_t inBa
                 lds_barrier();
 #pragma unroll
                 for (int k = 0; k < NB; ++k) {
-                    const BflyPos p = bfly_pos<RP, LGM>(tt + k * nt, LGC);
+                    const BflyPos p = bfly_pos<RP, LGM, E>(tt, k, nt, LGC);
 #pragma unroll
                     for (int i = 0; i < RP; ++i) x[k * RP + i] = cmul(x[k * RP + i], sRow[p.q + (i << lgMq)]);
                 }
@@ -691,7 +691,7 @@ __device__ __forceinline__ void stage0_pre(C* x, const FftPass& d, uint64_t inBa
                 }
 #pragma unroll
                 for (int k = 0; k < NB; ++k) {
-                    const BflyPos p = bfly_pos<RP, LGM>(tt + k * nt, LGC);
+                    const BflyPos p = bfly_pos<RP, LGM, E>(tt, k, nt, LGC);
                     const double m0 = (double)(2 * p.q + 1 - (1 << LGM));
                     const C e0 = unit_rev_fast(cvdv_frac(fma(gf.a, m0, gf.b)), R(0));
                     x[k * RP] = cmul(x[k * RP], e0);
@@ -747,7 +747,7 @@ __device__ __forceinline__ void last_store(C* __restrict__ out, const C* v, cons
     constexpr int lgMq = LGM - LGR;
 #pragma unroll
     for (int k = 0; k < NB; ++k) {
-        const BflyPos p = bfly_pos<RP, LGM>(tid + k * nt, LGC);
+        const BflyPos p = bfly_pos<RP, LGM, E>(tid, k, nt, LGC);
         const uint64_t g0 = outBase + ((uint64_t)p.hb << d.lgOutH2) + p.c;
 #pragma unroll
         for (int m = 0; m < RP; ++m) {
@@ -970,13 +970,14 @@ k_fft_tile(const typename CT<R>::type* in, typename CT<R>::type* out, FftPass d,
 // and d.conjOut before and after the next one.
 // The phases are evaluated at the natural index of the completed transform:
 // dD is the tile geometry seen in that index (row and row-block shifts), and
-// swapN > 0 exchanges the two swapN-bit digits at swapSh of the tile base (the
-// in-place L half leaves the register's digits exchanged).  Between the halves
-// the elements go through LDS from the last stage's order to stage 0's.
+// swapLo > 0 exchanges the digits of swapLo and swapHi bits at swapSh of the tile
+// base (the in-place L half leaves the register's digits exchanged).  Between the
+// halves the elements stay in their threads, reordered in registers.
 template <typename R, int LGM, int LGC, int E, bool STG>
 __global__ void __launch_bounds__((tile_threads_max<R, LGM, LGC>()))
 __attribute__((amdgpu_waves_per_eu((STG && sizeof(R) == 4) ? 8 : 1)))
-k_fft_fused(typename CT<R>::type* data, FftPass d, FftPass dD, FastDiag pre, int conjMid, int swapSh, int swapN,
+k_fft_fused(typename CT<R>::type* data, FftPass d, FftPass dD, FastDiag pre, int conjMid, int swapSh, int swapLo,
+            int swapHi,
             const typename CT<R>::type* __restrict__ tw, const typename CT<R>::type* __restrict__ tw4) {
     using C = typename CT<R>::type;
     constexpr int NST = Plan<LGM>::NST;
@@ -1015,10 +1016,10 @@ k_fft_fused(typename CT<R>::type* data, FftPass d, FftPass dD, FastDiag pre, int
     const uint64_t h1 = rr >> d.lgNH2Blk;
     const uint64_t base = (h1 << d.lgInH1) + ((h2Blk << d.lgHb) << d.lgInH2) + (loBlk << LGC);
     uint64_t natBase = base;
-    if (swapN > 0) {
-        const uint64_t m = (1ull << swapN) - 1ull;
-        const uint64_t lo = (base >> swapSh) & m, hi = (base >> (swapSh + swapN)) & m;
-        natBase = (base & ~(((m << swapN) | m) << swapSh)) | (((lo << swapN) | hi) << swapSh);
+    if (swapLo > 0) {
+        const uint64_t ml = (1ull << swapLo) - 1ull, mh = (1ull << swapHi) - 1ull;
+        const uint64_t lo = (base >> swapSh) & ml, hi = (base >> (swapSh + swapLo)) & mh;
+        natBase = (base & ~(((mh << swapLo) | ml) << swapSh)) | (((lo << swapHi) | hi) << swapSh);
     }
 
     C x[E];
@@ -1035,11 +1036,7 @@ k_fft_fused(typename CT<R>::type* data, FftPass d, FftPass dD, FastDiag pre, int
 #pragma unroll
         for (int i = 0; i < E; ++i) x[i].y = -x[i].y;
     }
-    // last stage's order -> stage 0's order
-    stage_write<RL, E, LGM, LGC, NST - 1>(lds, x, tid, nt);
-    lds_barrier();
-    stage_read<R0, E, LGM, LGC>(lds, x, tid, nt);
-    lds_barrier();
+    to_rows<LGM, E>(x);  // the last stage's order -> stage 0's
     // phases at the natural index, then the next transform's first half.  An
     // opaque copy of the thread id: index math derived from it (the store
     // addresses above all) would otherwise be computed early and held across
@@ -1287,8 +1284,9 @@ static void launch_pass(CVDVContext* ctx, const typename CT<R>::type* in, typena
 //   d1: transform over j2 (stride N1 S), columns (j1, lo), in place;
 //   d2: twiddle W_N^{j1 k2} on load, transform over j1 (stride S), row blocks
 //       k2, written transposed (k2 + N2 k1) out of place;
-// and, for equal digits, the in-place halves a pending transform completes with:
-//   dL:  d2 stored in place (momentum left with its digits exchanged);
+// and the in-place halves a pending transform completes with:
+//   dL:  d2 stored in place (momentum left with its digits exchanged: the low digit,
+//        n2 bits, above the high one, n1 bits);
 //   d1c: d1 with the twiddle W_N^{j1 j2} (j1 now the tile's) on load.
 struct FourStep {
     FftPass d1, d2, dL, d1c;
@@ -1320,12 +1318,10 @@ static bool four_step_geom(int prec, uint64_t total, int sh, int nb, FourStep& f
     f.d1c = f.d1;
     f.d1c.tw4 = 1; f.d1c.tw4Shift = sh; f.d1c.tw4HiBits = n1; f.d1c.tw4LogN = nb;
     f.d1c.tw4Uni = uni(f.d1c, sh, n1);
-    if (n1 == n2) {
-        PassGeom pL{(int)N1, S, N2, H, N * S, N1 * S, S, N * S, N1 * S, S};
-        f.hasL = fit_pass(pL, prec, f.dL, false, cfg);
-        f.dL.tw4 = 1; f.dL.tw4Shift = sh + n1; f.dL.tw4HiBits = n2; f.dL.tw4LogN = nb;
-        f.dL.tw4Uni = uni(f.dL, sh + n1, n2);
-    }
+    PassGeom pL{(int)N1, S, N2, H, N * S, N1 * S, S, N * S, N1 * S, S};
+    f.hasL = fit_pass(pL, prec, f.dL, false, cfg);
+    f.dL.tw4 = 1; f.dL.tw4Shift = sh + n1; f.dL.tw4HiBits = n2; f.dL.tw4LogN = nb;
+    f.dL.tw4Uni = uni(f.dL, sh + n1, n2);
     return true;
 }
 
@@ -1424,8 +1420,8 @@ static bool fft_run(CVDVContext* ctx, typename CT<R>::type* data, TmpFn tmpFn, u
 
 // ---------------------------------------------------------------- half transforms kept pending
 // Fused instances exist for digits of 2^FUSE_LGM_MIN .. 2^FUSE_LGM_MAX points
-// (registers of 2^10 .. 2^16 points).
-#define FUSE_LGM_MIN 5
+// (registers of 2^8 .. 2^16 points).
+#define FUSE_LGM_MIN 4
 #define FUSE_LGM_MAX 8
 
 // Every table of the program is read by row in tiles of geometry d (the test
@@ -1479,7 +1475,7 @@ static bool gen_affine_in_rows(const FastDiag& pre, int rowLo, int rowN) {
 
 template <typename R, int LGM, int LGC>
 static void launch_fused_geom(CVDVContext* ctx, typename CT<R>::type* data, const FftPass& d, const FftPass& dD,
-                              const FastDiag& pre, int conjMid, int swapSh, int swapN,
+                              const FastDiag& pre, int conjMid, int swapSh, int swapLo, int swapHi,
                               const typename CT<R>::type* tw, const typename CT<R>::type* tw4, uint64_t blocks,
                               int tile, size_t lds) {
     if constexpr (tile_instance<R, LGM, LGC>()) {
@@ -1495,12 +1491,12 @@ static void launch_fused_geom(CVDVContext* ctx, typename CT<R>::type* data, cons
             const bool gen = sizeof(R) == 8 || pre.ngen == 0 || dDg.genSteps;
             if (!dD.usePre || (tile_tables_by_row(pre, dD) && gen)) {
                 hipLaunchKernelGGL((k_fft_fused<R, LGM, LGC, 8, true>), dim3((unsigned)blocks), dim3(tile / 8), lds,
-                                   ctx->stream, data, d, dDg, pre, conjMid, swapSh, swapN, tw, tw4);
+                                   ctx->stream, data, d, dDg, pre, conjMid, swapSh, swapLo, swapHi, tw, tw4);
                 return;
             }
         }
         hipLaunchKernelGGL((k_fft_fused<R, LGM, LGC, 8, false>), dim3((unsigned)blocks), dim3(tile / 8), lds,
-                           ctx->stream, data, d, dDg, pre, conjMid, swapSh, swapN, tw, tw4);
+                           ctx->stream, data, d, dDg, pre, conjMid, swapSh, swapLo, swapHi, tw, tw4);
     } else {
         throw CvdvError{CVDV_ERR_UNSUPPORTED, "fused FFT tile shape without a kernel instance"};
     }
@@ -1508,12 +1504,12 @@ static void launch_fused_geom(CVDVContext* ctx, typename CT<R>::type* data, cons
 
 template <typename R, int LGM>
 static void launch_fused_lgm(CVDVContext* ctx, typename CT<R>::type* data, const FftPass& d, const FftPass& dD,
-                             const FastDiag& pre, int conjMid, int swapSh, int swapN,
+                             const FastDiag& pre, int conjMid, int swapSh, int swapLo, int swapHi,
                              const typename CT<R>::type* tw, const typename CT<R>::type* tw4, uint64_t blocks,
                              int tile, size_t lds) {
     switch (d.lgC) {
 #define CVDV_FUSE_C(L) \
-    case L: launch_fused_geom<R, LGM, L>(ctx, data, d, dD, pre, conjMid, swapSh, swapN, tw, tw4, blocks, tile, lds); break;
+    case L: launch_fused_geom<R, LGM, L>(ctx, data, d, dD, pre, conjMid, swapSh, swapLo, swapHi, tw, tw4, blocks, tile, lds); break;
         CVDV_FUSE_C(0) CVDV_FUSE_C(1) CVDV_FUSE_C(2) CVDV_FUSE_C(3) CVDV_FUSE_C(4) CVDV_FUSE_C(5)
 #undef CVDV_FUSE_C
         default: throw CvdvError{CVDV_ERR_UNSUPPORTED, "fused FFT tile column count out of range"};
@@ -1522,7 +1518,7 @@ static void launch_fused_lgm(CVDVContext* ctx, typename CT<R>::type* data, const
 
 template <typename R>
 static void launch_fused(CVDVContext* ctx, const FftPass& d, const FftPass& dD, const FastDiag& pre, int conjMid,
-                         int swapSh, int swapN, uint64_t nH1) {
+                         int swapSh, int swapLo, int swapHi, uint64_t nH1) {
     using C = typename CT<R>::type;
     const int prec = ctx->prec;
     const C* tw = (const C*)stage_table(ctx, d.lgM, prec);
@@ -1536,8 +1532,8 @@ static void launch_fused(CVDVContext* ctx, const FftPass& d, const FftPass& dD, 
     const int pid = prof_begin(ctx, KK_FFT_FUSED);
     switch (d.lgM) {
 #define CVDV_FUSE_M(L) \
-    case L: launch_fused_lgm<R, L>(ctx, data, dd, dD, pre, conjMid, swapSh, swapN, tw, tw4, blocks, tile, lds); break;
-        CVDV_FUSE_M(5) CVDV_FUSE_M(6) CVDV_FUSE_M(7) CVDV_FUSE_M(8)
+    case L: launch_fused_lgm<R, L>(ctx, data, dd, dD, pre, conjMid, swapSh, swapLo, swapHi, tw, tw4, blocks, tile, lds); break;
+        CVDV_FUSE_M(4) CVDV_FUSE_M(5) CVDV_FUSE_M(6) CVDV_FUSE_M(7) CVDV_FUSE_M(8)
 #undef CVDV_FUSE_M
         default: throw CvdvError{CVDV_ERR_UNSUPPORTED, "fused FFT digit length out of range"};
     }
@@ -1547,11 +1543,14 @@ static void launch_fused(CVDVContext* ctx, const FftPass& d, const FftPass& dD, 
 
 static uint64_t bit_field(int sh, int n) { return n > 0 ? (((1ull << n) - 1ull) << sh) : 0ull; }
 
-// The four-step of this register can leave halves pending: equal digits, fused
-// instances for the digit length, and tiles that store straight to global memory.
+// The four-step of this register can leave halves pending: fused instances for both
+// digits, and tiles that store straight to global memory.  The digits may differ: the
+// halves of one transform alternate between them, and a fused pass (L of one transform
+// and H of the next, whose high digit is the momentum's, or the twiddle and H of one and
+// H of the next) always runs over one digit.
 static bool fusable(const CVDVContext* ctx, const FourStep& f, int nb, const FftCfg& cfg) {
-    return ctx->fuseFt && cfg.fuse != 0 && !ctx->rec && f.n1 == f.n2 && f.n1 >= FUSE_LGM_MIN && f.n1 <= FUSE_LGM_MAX && f.hasL &&
-           f.d1.directOut && f.dL.directOut && nb == 2 * f.n1;
+    return ctx->fuseFt && cfg.fuse != 0 && !ctx->rec && f.n1 >= FUSE_LGM_MIN && f.n2 <= FUSE_LGM_MAX && f.hasL &&
+           f.d1.directOut && f.dL.directOut && nb == f.n1 + f.n2;
 }
 
 // Complete the half-done transform D (its record already cleared).
@@ -1626,7 +1625,6 @@ static bool fft_deferred(CVDVContext* ctx, int sh, int nb, bool inverse, const D
     }
     FourStep f;
     if (!four_step_geom(ctx->prec, total, sh, nb, f, cfg) || !fusable(ctx, f, nb, cfg)) return false;
-    const int n = f.n1;
     bool act = false, folded = false;
     if (FtDefer* rec = ctx->defer.find(sh)) {
         FtDefer& D = *rec;
@@ -1635,8 +1633,8 @@ static bool fft_deferred(CVDVContext* ctx, int sh, int nb, bool inverse, const D
         FftPass d = high ? f.d1c : f.dL;
         FftPass dD = d;  // the tile in the natural index of the completed transform
         if (!high) {
-            dD.lgInR = sh + n;   // rows: the lo digit here is the momentum's hi digit
-            dD.lgInH2 = sh;      // row blocks: the hi digit here is the momentum's lo digit
+            dD.lgInR = sh + f.n2;  // rows: the lo digit here is the momentum's hi digit
+            dD.lgInH2 = sh;        // row blocks: the hi digit here is the momentum's lo digit
         }
         const uint64_t natBits = tile_bits(dD);
         const double scale = outScale * D.scale;
@@ -1651,7 +1649,7 @@ static bool fft_deferred(CVDVContext* ctx, int sh, int nb, bool inverse, const D
             dD.tw4 = 0;
             dD.usePre = act ? 1 : 0;
             dD.conjIn = inverse ? 1 : 0;
-            launch_fused<R>(ctx, d, dD, pre, D.inv, sh, high ? 0 : n, f.H);
+            launch_fused<R>(ctx, d, dD, pre, D.inv, sh, high ? 0 : f.n1, high ? 0 : f.n2, f.H);
             D = FtDefer{1, sh, nb, high ? 0 : 1, inverse ? 1 : 0, 1.0};
             return true;
         }

@@ -121,11 +121,9 @@ __device__ __forceinline__ C chain_apply(const ChainStep& st, double rev, C v) {
     return cmk<C>(p.x, p.y);
 }
 
-// A thread owns the rows q + j M/8, j < 8, of one column and block, in every stage: the
-// butterfly k of a last stage of radix RL = 8/NB holds the rows q + (M/8) (k + NB m), so
-// its outputs, reordered in registers, are the next transform's first inputs and no
-// exchange is needed between transforms.  Each block of rows is transformed by threads
-// and LDS of its own.
+// A thread owns the rows q + j M/8, j < 8, of one column and block in every stage
+// (bfly_pos), so no exchange is needed between transforms.  Each block of rows is
+// transformed by threads and LDS of its own.
 // The steps are read from the kernel's argument segment straight into LDS (a is the
 // first argument): indexing the argument at run time would copy it to scratch memory.
 template <typename R, int LGM, int LGC> constexpr int chain_threads_max() { return LGM + LGC >= 13 ? 1024 : 512; }
@@ -133,8 +131,7 @@ template <typename R, int LGM, int LGC>
 __global__ void __launch_bounds__((chain_threads_max<R, LGM, LGC>()), 4)
 k_fft_chain(ChainArgs a, typename CT<R>::type* data, const typename CT<R>::type* __restrict__ tw) {
     using C = typename CT<R>::type;
-    constexpr int NST = Plan<LGM>::NST, EX = chain_ex<R, LGC>();
-    constexpr int RL = 1 << Plan<LGM>::lgr(NST - 1), NB = 8 / RL;
+    constexpr int EX = chain_ex<R, LGC>();
     constexpr int M = 1 << LGM, ST = 1 << (LGM + LGC - 3);  // threads of a block
     extern __shared__ __align__(16) unsigned char smem_raw[];
     __shared__ ChainStep steps[FT_CHAIN_MAX];
@@ -218,15 +215,10 @@ k_fft_chain(ChainArgs a, typename CT<R>::type* data, const typename CT<R>::type*
         }
         stage_compute<8, 8, LGM, LGC, 0, false>(x, tw, ti, ST);
         run_stages<LGM, LGC, 1, 8, false, EX>(x, lds, tw, ti, ST);
-        C y[8];
+        to_rows<LGM, 8>(x);
+        if (inv) {
 #pragma unroll
-        for (int k = 0; k < NB; ++k)
-#pragma unroll
-            for (int m = 0; m < RL; ++m) y[k + NB * m] = x[k * RL + m];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            x[j] = y[j];
-            if (inv) x[j].y = -x[j].y;
+            for (int j = 0; j < 8; ++j) x[j].y = -x[j].y;
         }
     }
 #pragma unroll

@@ -72,24 +72,52 @@ template <int LGM> struct SplitPlan {
     static constexpr int total() { return off(Plan<LGM>::NST); }
 };
 
-// Stockham stage geometry.  Butterfly b of a stage of radix RP (sub-length
-// L = 2^lgL already transformed) takes rows q + i*M/RP of column c in block hb
-// and writes rows ob + m*L, ob = hb*M + (q/L)*RP*L + (q mod L); every thread
-// owns E/RP butterflies b = tid + k*nt.
+// Stockham stage geometry.  A butterfly of a stage of radix RP (sub-length L = 2^lgL
+// already transformed) takes rows q + i*M/RP of column c in block hb and writes rows
+// ob + m*L, ob = hb*M + (q/L)*RP*L + (q mod L); every thread owns E/RP butterflies.
 struct BflyPos {
     int c, q, hb;
 };
 
-template <int RP, int LGM>
-__device__ __forceinline__ BflyPos bfly_pos(int b, int lgC) {
+// The thread's butterfly k.  Where a column has at least E rows the thread owns the rows
+// q0 + j M/E, j < E, of its column and block in every stage (butterfly k sits at
+// q0 + k M/E), so a last stage's outputs, reordered in registers (to_rows), are a first
+// stage's inputs; shorter columns deal the butterflies out nt apart.
+template <int RP, int LGM, int E>
+__device__ __forceinline__ BflyPos bfly_pos(int tid, int k, int nt, int lgC) {
     constexpr int LGR = RP == 8 ? 3 : (RP == 4 ? 2 : 1);
-    constexpr int lgMq = LGM - LGR;
+    constexpr int LGE = E == 16 ? 4 : 3;
+    static_assert(E == 8 || E == 16, "elements of a thread");
     BflyPos p;
-    p.c = b & ((1 << lgC) - 1);
-    const int rest = b >> lgC;
-    p.q = rest & ((1 << lgMq) - 1);
-    p.hb = rest >> lgMq;
+    if constexpr (LGM >= LGE) {
+        p.c = tid & ((1 << lgC) - 1);
+        const int rest = tid >> lgC;
+        p.q = (rest & ((1 << (LGM - LGE)) - 1)) + k * (1 << (LGM - LGE));
+        p.hb = rest >> (LGM - LGE);
+    } else {
+        constexpr int lgMq = LGM - LGR;
+        const int b = tid + k * nt;
+        p.c = b & ((1 << lgC) - 1);
+        const int rest = b >> lgC;
+        p.q = rest & ((1 << lgMq) - 1);
+        p.hb = rest >> lgMq;
+    }
     return p;
+}
+
+// Outputs of a last stage (butterfly k, output m: row q0 + (k + NB m) M/E) in the order of
+// the thread's rows.
+template <int LGM, int E, typename C>
+__device__ __forceinline__ void to_rows(C* x) {
+    constexpr int RL = LGM % 3 == 0 ? 8 : 1 << (LGM % 3), NB = E / RL;
+    static_assert((1 << LGM) >= E, "columns of at least E rows");
+    C y[E];
+#pragma unroll
+    for (int k = 0; k < NB; ++k)
+#pragma unroll
+        for (int m = 0; m < RL; ++m) y[k + NB * m] = x[k * RL + m];
+#pragma unroll
+    for (int j = 0; j < E; ++j) x[j] = y[j];
 }
 
 // Twiddle the inputs of the butterflies in x (stage S, radix RP) and transform.
@@ -103,7 +131,7 @@ __device__ __forceinline__ void stage_compute(C* x, const C* __restrict__ tw, in
 #pragma unroll
     for (int k = 0; k < NB; ++k) {
         if (lgL > 0) {
-            const BflyPos p = bfly_pos<RP, LGM>(tid + k * nt, lgC);
+            const BflyPos p = bfly_pos<RP, LGM, E>(tid, k, nt, lgC);
             const int pq = p.q & ((1 << lgL) - 1);
             if constexpr (!TWL) {
                 const C* t = tw + Plan<LGM>::off(S) + pq * (RP - 1);
@@ -135,7 +163,7 @@ __device__ __forceinline__ void last_twiddles(C* w, const C* __restrict__ tw, in
     constexpr int S = Plan<LGM>::NST - 1, RP = 1 << Plan<LGM>::lgr(S);
 #pragma unroll
     for (int k = 0; k < E / RP; ++k) {
-        const C* t = tw + Plan<LGM>::off(S) + bfly_pos<RP, LGM>(tid + k * nt, 0).q * (RP - 1);
+        const C* t = tw + Plan<LGM>::off(S) + bfly_pos<RP, LGM, E>(tid, k, nt, 0).q * (RP - 1);
 #pragma unroll
         for (int i = 1; i < RP; ++i) w[k * (RP - 1) + i - 1] = t[i - 1];
     }
@@ -160,7 +188,7 @@ __device__ __forceinline__ void stage_write(C* lds, const C* x, int tid, int nt)
     constexpr int STRIDE = 1 << (lgL + LGC);
 #pragma unroll
     for (int k = 0; k < NB; ++k) {
-        const BflyPos p = bfly_pos<RP, LGM>(tid + k * nt, LGC);
+        const BflyPos p = bfly_pos<RP, LGM, E>(tid, k, nt, LGC);
         const int ob = (p.hb << LGM) + ((p.q >> lgL) << (LGR + lgL)) + (p.q & ((1 << lgL) - 1));
         const int i0 = (ob << LGC) + p.c, pb = lay_ix<LAY>(i0);
         if constexpr (LAY == 1 || LAY == 2 || (LAY == 3 && S == 0)) {
@@ -185,7 +213,7 @@ __device__ __forceinline__ void stage_read(const C* lds, C* x, int tid, int nt) 
     constexpr int STRIDE = 1 << (lgMq + LGC);
 #pragma unroll
     for (int k = 0; k < NB; ++k) {
-        const BflyPos p = bfly_pos<RP, LGM>(tid + k * nt, LGC);
+        const BflyPos p = bfly_pos<RP, LGM, E>(tid, k, nt, LGC);
         const int i0 = (((p.hb << LGM) + p.q) << LGC) + p.c, pb = lay_ix<LAY>(i0);
 #pragma unroll
         for (int i = 0; i < RP; ++i) x[k * RP + i] = lds[lds_at<STRIDE, LAY>(i0, pb, i)];

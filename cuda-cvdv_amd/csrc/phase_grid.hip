@@ -159,7 +159,7 @@ k_grid_rows(double2* __restrict__ A, const double2* __restrict__ spec, uint64_t 
         step[e] = unit_rev(cvdv_frac(0.125 * (double)(i < 4 ? i : i - 8) * t), 0.0);
     }
     __syncthreads();
-    const BflyPos p0 = bfly_pos<8, LGM>(tid, 0);
+    const BflyPos p0 = bfly_pos<8, LGM, 8>(tid, 0, NT, 0);
     const uint64_t myRow = row0 + p0.hb;
     const double myT = myRow < rows ? tx[perSlice ? myRow % nxa : myRow] : 0.0;
     const double2 u0 = unit_rev(cvdv_frac((double)p0.q * myT * (1.0 / N)), 0.0);

@@ -325,7 +325,7 @@ k_wigner_rows(void* __restrict__ outv, const C* __restrict__ X, uint64_t S, int 
     const double w = dx / PI;
 #pragma unroll
     for (int k = 0; k < 8 / RL; ++k) {
-        const BflyPos p = bfly_pos<RL, LGM>(tid + k * NT, 0);
+        const BflyPos p = bfly_pos<RL, LGM, 8>(tid, k, NT, 0);
         const bool n0 = bad[2 * p.hb] != 0, n1 = bad[2 * p.hb + 1] != 0;
         if (2 * (a0 + p.hb) >= N) continue;
 #pragma unroll
@@ -363,7 +363,7 @@ k_husimi_rows(double* __restrict__ acc, const C* __restrict__ X, uint64_t S, int
     double w[8], sum[8];
 #pragma unroll
     for (int k = 0; k < 8 / R0; ++k) {
-        const BflyPos p = bfly_pos<R0, LGM>(tid + k * NT, 0);
+        const BflyPos p = bfly_pos<R0, LGM, 8>(tid, k, NT, 0);
 #pragma unroll
         for (int i = 0; i < R0; ++i) {
             const double d = ((double)(p.q + i * (N / R0)) - (double)(q0 + p.hb)) * dx;
@@ -382,7 +382,7 @@ k_husimi_rows(double* __restrict__ acc, const C* __restrict__ X, uint64_t S, int
         double2 x[8];
 #pragma unroll
         for (int k = 0; k < 8 / R0; ++k) {
-            const BflyPos p = bfly_pos<R0, LGM>(ti + k * NT, 0);
+            const BflyPos p = bfly_pos<R0, LGM, 8>(ti, k, NT, 0);
 #pragma unroll
             for (int i = 0; i < R0; ++i) x[k * R0 + i] = slice_at(X, s, LGM, p.q + i * (N / R0), refl);
         }
@@ -395,7 +395,7 @@ k_husimi_rows(double* __restrict__ acc, const C* __restrict__ X, uint64_t S, int
     }
 #pragma unroll
     for (int k = 0; k < 8 / RL; ++k) {
-        const BflyPos p = bfly_pos<RL, LGM>(tid + k * NT, 0);
+        const BflyPos p = bfly_pos<RL, LGM, 8>(tid, k, NT, 0);
         if (q0 + p.hb >= N) continue;
 #pragma unroll
         for (int m = 0; m < RL; ++m) acc[(uint64_t)(q0 + p.hb) * N + p.q + m * (N / RL)] = sum[k * RL + m];

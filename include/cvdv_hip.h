@@ -100,7 +100,7 @@ void   cvdvSynchronize(CVDVContext* ctx);
  * layout (both are otherwise applied lazily by the next kernel). */
 void   cvdvFlush(CVDVContext* ctx);
 /* Consecutive Fourier transforms of one register that the four-step split
- * serves (registers of 2^10 .. 2^16 points whose tile does not hold them whole)
+ * serves (registers of 2^8 .. 2^16 points whose tile does not hold them whole)
  * share HBM passes: each transform runs as two half passes, and the second half
  * of one is fused with the first half of the next, the phases between them
  * applied in the same pass (m transforms: m + 1 passes instead of 2m).  on = 0
