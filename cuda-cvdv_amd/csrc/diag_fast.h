@@ -24,6 +24,7 @@
 #pragma once
 
 #include "cvdv_internal.h"
+#include "phase_eval.h"
 
 #define CVDV_FAST_TABS 6
 #define CVDV_FAST_GEN 4
@@ -107,6 +108,32 @@ template <typename C>
 __device__ __forceinline__ C apply_fast(const FastDiag& f, uint64_t g, C v) {
     return cmul(v, fast_factor<C>(f, g));
 }
+
+// A program whose terms are all generic (inplace_diag), at element g, in FP64: for small
+// states, where the launch that builds tables costs more than evaluating the terms.
+template <typename C>
+__device__ __forceinline__ double2 inplace_factor(const FastDiag& f, uint64_t g) {
+    using R = decltype(C{}.x);
+    double r = f.genrev;
+#pragma unroll
+    for (int i = 0; i < CVDV_FAST_GEN; ++i)
+        if (i < f.ngen) r += cvdv_frac(diag_term_rev(f.gen[i], g));
+    return unit_turn(cvdv_frac(r), R(0));
+}
+
+// Element g of the state in FP64, the pending phases applied (IN: an inplace_diag
+// program; a complex64 element is not rounded in between).
+template <bool IN, typename C>
+__device__ __forceinline__ double2 phased(const FastDiag& f, int usep, uint64_t g, C v) {
+    if (!usep) return make_double2((double)v.x, (double)v.y);
+    if constexpr (IN) return cmul(make_double2((double)v.x, (double)v.y), inplace_factor<C>(f, g));
+    const C w = apply_fast(f, g, v);
+    return make_double2((double)w.x, (double)w.y);
+}
+
+// Host side (gates.hip): the program evaluated in place; false when it is not for the
+// context's state size or has too many terms (compile_diag then).
+bool inplace_diag(const CVDVContext* ctx, const DiagProg& p, FastDiag& f, bool& active);
 
 // Host side (gates.hip): build the tables on ctx->stream and return the
 // compiled program; `active` is false when the program is the identity.

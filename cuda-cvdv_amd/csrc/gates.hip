@@ -11,6 +11,7 @@
 #include <cmath>
 #include <cstdio>
 #include <string>
+#include <type_traits>
 
 #include "cvdv_internal.h"
 #include "diag_fast.h"
@@ -24,7 +25,8 @@ static const double SQRT2 = 1.41421356237309504880;
 // per iteration, their loads issued together.
 #define PAIRS_PER_THREAD 4
 
-template <typename C>
+// IN (here and below): the program is evaluated in place (inplace_diag).
+template <typename C, bool IN>
 __global__ void k_diag(C* __restrict__ s, uint64_t total, FastDiag f) {
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t g0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; g0 < total; g0 += PAIRS_PER_THREAD * stride) {
@@ -34,7 +36,10 @@ __global__ void k_diag(C* __restrict__ s, uint64_t total, FastDiag f) {
             if (g0 + k * stride < total) v[k] = s[g0 + k * stride];
 #pragma unroll
         for (int k = 0; k < PAIRS_PER_THREAD; ++k)
-            if (g0 + k * stride < total) s[g0 + k * stride] = apply_fast(f, g0 + k * stride, v[k]);
+            if (g0 + k * stride < total) {
+                const double2 w = phased<IN>(f, 1, g0 + k * stride, v[k]);
+                s[g0 + k * stride] = cmk<C>(w.x, w.y);
+            }
     }
 }
 
@@ -112,7 +117,7 @@ __global__ void k_make_tables(C* __restrict__ arena, TabMakeArgs a) {
 // 2x2 unitary on the pair (bit = 0, bit = 1); pending phases applied on load.
 // The matrix product runs in FP64 for both precisions, so a complex64 state is
 // rounded once per gate and never sees a rounded (non-unitary) matrix.
-template <typename C>
+template <typename C, bool IN>
 __global__ void k_qubit(C* __restrict__ s, uint64_t npairs, int bit, double2 m00, double2 m01,
                         double2 m10, double2 m11, FastDiag p, int usep) {
     const uint64_t lowmask = (1ull << bit) - 1ull;
@@ -137,13 +142,7 @@ __global__ void k_qubit(C* __restrict__ s, uint64_t npairs, int bit, double2 m00
             if (pid >= npairs) continue;
             const uint64_t i0 = ((pid & ~lowmask) << 1) | (pid & lowmask);
             const uint64_t i1 = i0 | (1ull << bit);
-            C va = a[k], vb = b[k];
-            if (usep) {
-                va = apply_fast(p, i0, va);
-                vb = apply_fast(p, i1, vb);
-            }
-            const double2 ad = make_double2((double)va.x, (double)va.y);
-            const double2 bd = make_double2((double)vb.x, (double)vb.y);
+            const double2 ad = phased<IN>(p, usep, i0, a[k]), bd = phased<IN>(p, usep, i1, b[k]);
             const double2 t00 = cmul(m00, ad), t01 = cmul(m01, bd), t10 = cmul(m10, ad), t11 = cmul(m11, bd);
             s[i0] = cmk<C>(t00.x + t01.x, t00.y + t01.y);
             s[i1] = cmk<C>(t10.x + t11.x, t10.y + t11.y);
@@ -154,7 +153,7 @@ __global__ void k_qubit(C* __restrict__ s, uint64_t npairs, int bit, double2 m00
 // Conditional reflection j <-> N-1-j of the field [sh, sh+nb) where the
 // control bit of the logically lower partner is 1 (reference semantics,
 // src/cuda/kernels/gates.cuh:134-157 and torchCvdv.py:122-137).
-template <typename C>
+template <typename C, bool IN>
 __global__ void k_cparity(C* __restrict__ s, uint64_t npairs, int sh, int nb, int ctrlPos,
                           int ctrlFlip, int tgtRefl, FastDiag p, int usep) {
     const int top = sh + nb - 1;
@@ -181,8 +180,9 @@ __global__ void k_cparity(C* __restrict__ s, uint64_t npairs, int sh, int nb, in
             const uint64_t i1 = i0 ^ fmask;
             C va = a[k], vb = b[k];
             if (usep) {
-                va = apply_fast(p, i0, va);
-                vb = apply_fast(p, i1, vb);
+                const double2 pa = phased<IN>(p, 1, i0, va), pb = phased<IN>(p, 1, i1, vb);
+                va = cmk<C>(pa.x, pa.y);
+                vb = cmk<C>(pb.x, pb.y);
             }
             const uint64_t lower = tgtRefl ? i1 : i0;
             const int cb = (int)((lower >> ctrlPos) & 1ull) ^ ctrlFlip;
@@ -487,6 +487,38 @@ FastDiag compile_diag(CVDVContext* ctx, const DiagProg& p, bool& active, double 
     return f;
 }
 
+// Up to 2^20 amplitudes a table build (3 to 4.5 us) costs more than evaluating a
+// program's terms where they are read: 2 us at 2^20, 4 at 2^21 (complex128, two terms).
+#define INPLACE_LG_MAX 20
+
+bool inplace_diag(const CVDVContext* ctx, const DiagProg& p, FastDiag& f, bool& active) {
+    if (ctx->totalQbt > INPLACE_LG_MAX) return false;
+    f = FastDiag{};
+    for (int i = 0; i < p.n; ++i) {
+        if (term_is_identity(p.t[i])) continue;
+        if (f.ngen == CVDV_FAST_GEN) return false;
+        f.gen[f.ngen++] = p.t[i];
+    }
+    f.genrev = cvdv_frac(p.grev);
+    active = f.ngen > 0 || f.genrev != 0.0;
+    return true;
+}
+
+// A kernel over the pairs (or elements) of the state with the program p applied: go(IN,
+// program, active, pairs a thread).  Evaluated in place one pair a thread is enough work,
+// and spreads small states over more of the chip.
+template <typename F>
+static void with_program(CVDVContext* ctx, const DiagProg& p, F go) {
+    FastDiag f;
+    bool act;
+    if (inplace_diag(ctx, p, f, act)) {
+        go(std::true_type{}, f, act, 1);
+    } else {
+        f = compile_diag(ctx, p, act);
+        go(std::false_type{}, f, act, PAIRS_PER_THREAD);
+    }
+}
+
 // Bits of the flat index a term depends on.
 static uint64_t term_bits(const DiagTerm& t) {
     auto field = [](int sh, int nb) { return (((uint64_t)1 << nb) - 1ull) << sh; };
@@ -571,17 +603,17 @@ void launch_diag(CVDVContext* ctx, const DiagProg& pp) {
     chain_flush(ctx);
     fft_settle_for(ctx, pp);
     const uint64_t n = ctx->totalSize;
-    bool act;
-    const FastDiag p = compile_diag(ctx, pp, act);
-    const int pid = prof_begin(ctx, KK_DIAG);
-    if (ctx->prec == CVDV_C128)
-        hipLaunchKernelGGL(k_diag<double2>, dim3(grid_for((n + PAIRS_PER_THREAD - 1) / PAIRS_PER_THREAD)), dim3(256), 0, ctx->stream,
-                           (double2*)ctx->state(), n, p);
-    else
-        hipLaunchKernelGGL(k_diag<float2>, dim3(grid_for((n + PAIRS_PER_THREAD - 1) / PAIRS_PER_THREAD)), dim3(256), 0, ctx->stream,
-                           (float2*)ctx->state(), n, p);
-    HIPCHK(hipGetLastError());
-    prof_end(ctx, pid);
+    with_program(ctx, pp, [&](auto in, const FastDiag& p, bool, int per) {
+        constexpr bool IN = decltype(in)::value;
+        const dim3 grid(grid_for((n + per - 1) / per));
+        const int pid = prof_begin(ctx, KK_DIAG);
+        if (ctx->prec == CVDV_C128)
+            hipLaunchKernelGGL((k_diag<double2, IN>), grid, dim3(256), 0, ctx->stream, (double2*)ctx->state(), n, p);
+        else
+            hipLaunchKernelGGL((k_diag<float2, IN>), grid, dim3(256), 0, ctx->stream, (float2*)ctx->state(), n, p);
+        HIPCHK(hipGetLastError());
+        prof_end(ctx, pid);
+    });
 }
 
 void ctx_flush(CVDVContext* ctx) {
@@ -738,21 +770,23 @@ static void qubit_gate(CVDVContext* ctx, int reg, int qubit, const double m[8]) 
     fft_settle_bits(ctx, 1ull << bit);
     const DiagProg taken = ctx_take_involving(ctx, 1ull << bit);
     fft_settle_for(ctx, taken);
-    bool act;
-    const FastDiag p = compile_diag(ctx, taken, act);
-    const int usep = act ? 1 : 0;
     const uint64_t np = ctx->totalSize / 2;
     const double2 m00 = make_double2(mm[0], mm[1]), m01 = make_double2(mm[2], mm[3]);
     const double2 m10 = make_double2(mm[4], mm[5]), m11 = make_double2(mm[6], mm[7]);
-    const int pid = prof_begin(ctx, KK_QUBIT);
-    if (ctx->prec == CVDV_C128)
-        hipLaunchKernelGGL(k_qubit<double2>, dim3(grid_for((np + PAIRS_PER_THREAD - 1) / PAIRS_PER_THREAD)), dim3(256), 0, ctx->stream,
-                           (double2*)ctx->state(), np, bit, m00, m01, m10, m11, p, usep);
-    else
-        hipLaunchKernelGGL(k_qubit<float2>, dim3(grid_for((np + PAIRS_PER_THREAD - 1) / PAIRS_PER_THREAD)), dim3(256), 0, ctx->stream,
-                           (float2*)ctx->state(), np, bit, m00, m01, m10, m11, p, usep);
-    HIPCHK(hipGetLastError());
-    prof_end(ctx, pid);
+    with_program(ctx, taken, [&](auto in, const FastDiag& p, bool act, int per) {
+        constexpr bool IN = decltype(in)::value;
+        const dim3 grid(grid_for((np + per - 1) / per));
+        const int usep = act ? 1 : 0;
+        const int pid = prof_begin(ctx, KK_QUBIT);
+        if (ctx->prec == CVDV_C128)
+            hipLaunchKernelGGL((k_qubit<double2, IN>), grid, dim3(256), 0, ctx->stream, (double2*)ctx->state(), np,
+                               bit, m00, m01, m10, m11, p, usep);
+        else
+            hipLaunchKernelGGL((k_qubit<float2, IN>), grid, dim3(256), 0, ctx->stream, (float2*)ctx->state(), np,
+                               bit, m00, m01, m10, m11, p, usep);
+        HIPCHK(hipGetLastError());
+        prof_end(ctx, pid);
+    });
 }
 
 static void zbit(CVDVContext* ctx, int reg, int qubit, double theta) {
@@ -809,21 +843,21 @@ static void cparity(CVDVContext* ctx, int tgt, int creg, int cq) {
     fft_settle_bits(ctx, ((((uint64_t)1 << nb) - 1ull) << ctx->pshift[tgt]) | (1ull << cpos));
     const DiagProg taken = ctx_take_involving(ctx, (((uint64_t)1 << nb) - 1ull) << ctx->pshift[tgt]);
     fft_settle_for(ctx, taken);
-    bool act;
-    const FastDiag p = compile_diag(ctx, taken, act);
-    const int usep = act ? 1 : 0;
     const uint64_t np = ctx->totalSize / 2;
-    const int pid = prof_begin(ctx, KK_CPARITY);
-    if (ctx->prec == CVDV_C128)
-        hipLaunchKernelGGL(k_cparity<double2>, dim3(grid_for((np + PAIRS_PER_THREAD - 1) / PAIRS_PER_THREAD)), dim3(256), 0, ctx->stream,
-                           (double2*)ctx->state(), np, ctx->pshift[tgt], nb, cpos, ctx->refl[creg],
-                           ctx->refl[tgt], p, usep);
-    else
-        hipLaunchKernelGGL(k_cparity<float2>, dim3(grid_for((np + PAIRS_PER_THREAD - 1) / PAIRS_PER_THREAD)), dim3(256), 0, ctx->stream,
-                           (float2*)ctx->state(), np, ctx->pshift[tgt], nb, cpos, ctx->refl[creg],
-                           ctx->refl[tgt], p, usep);
-    HIPCHK(hipGetLastError());
-    prof_end(ctx, pid);
+    with_program(ctx, taken, [&](auto in, const FastDiag& p, bool act, int per) {
+        constexpr bool IN = decltype(in)::value;
+        const dim3 grid(grid_for((np + per - 1) / per));
+        const int usep = act ? 1 : 0;
+        const int pid = prof_begin(ctx, KK_CPARITY);
+        if (ctx->prec == CVDV_C128)
+            hipLaunchKernelGGL((k_cparity<double2, IN>), grid, dim3(256), 0, ctx->stream, (double2*)ctx->state(), np,
+                               ctx->pshift[tgt], nb, cpos, ctx->refl[creg], ctx->refl[tgt], p, usep);
+        else
+            hipLaunchKernelGGL((k_cparity<float2, IN>), grid, dim3(256), 0, ctx->stream, (float2*)ctx->state(), np,
+                               ctx->pshift[tgt], nb, cpos, ctx->refl[creg], ctx->refl[tgt], p, usep);
+        HIPCHK(hipGetLastError());
+        prof_end(ctx, pid);
+    });
 }
 
 static void swap_regs(CVDVContext* ctx, int r1, int r2) {
