@@ -202,53 +202,99 @@ __global__ void k_from_c128(C* __restrict__ out, const double2* __restrict__ in,
         out[g] = cmk<C>(in[g].x, in[g].y);
 }
 
-struct LayoutArgs {
-    int pshift[CVDV_MAX_REG];
-    int flw[CVDV_MAX_REG];
-    int nq[CVDV_MAX_REG];
-    int refl[CVDV_MAX_REG];
+// Where physical index bits go in the canonical order: perm(g) ^ flip, perm moving each
+// register's field from its physical shift to its canonical one.  A move goes through
+// tiles over nb index bits: pos (physical, ascending) holds the lowest physical bits, so
+// a tile is read in runs, and the bits that land lowest in the canonical order, so it is
+// written in runs; ord lists the tile's bits by canonical position.
+#define MOVE_TILE_BITS 10
+struct MoveArgs {
+    uint64_t rest;  // physical bits outside the tile
+    uint64_t flip;
+    int nb;
+    int pos[MOVE_TILE_BITS], cpos[MOVE_TILE_BITS], ord[MOVE_TILE_BITS];
     int nreg;
+    int pshift[CVDV_MAX_REG], flw[CVDV_MAX_REG], nq[CVDV_MAX_REG];
 };
 
-__device__ __forceinline__ uint64_t canon_index(const LayoutArgs& L, uint64_t g) {
-    uint64_t o = 0;
-    for (int r = 0; r < L.nreg; ++r) {
-        const uint64_t mask = (1ull << L.nq[r]) - 1ull;
-        uint64_t j = (g >> L.pshift[r]) & mask;
-        if (L.refl[r]) j = mask - j;
-        o |= j << L.flw[r];
-    }
-    return o;
-}
-
-// out[canonical(g)] = pending(g) * in[g]
-template <typename C>
-__global__ void k_materialize(C* __restrict__ out, const C* __restrict__ in, uint64_t total,
-                              LayoutArgs L, DiagProg p) {
-    for (uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; g < total;
-         g += (uint64_t)gridDim.x * blockDim.x) {
-        C v = in[g];
-        if (p.n || p.grev != 0.0) v = apply_diag(p, g, v);
-        out[canon_index(L, g)] = v;
+// Where an element of the result goes.
+enum { OUT_STATE = 0, OUT_C128 = 1, OUT_SPLIT = 2 };  // the state's type, complex128, planes re | im
+template <int OUT, typename C>
+__device__ __forceinline__ void put_out(void* out, uint64_t total, uint64_t o, double2 v) {
+    if constexpr (OUT == OUT_STATE) {
+        ((C*)out)[o] = cmk<C>(v.x, v.y);
+    } else if constexpr (OUT == OUT_C128) {
+        ((double2*)out)[o] = v;
+    } else {
+        ((double*)out)[o] = v.x;
+        ((double*)out)[total + o] = v.y;
     }
 }
 
-template <typename C>
-__global__ void k_split(double* __restrict__ re, double* __restrict__ im, const C* __restrict__ in,
-                        uint64_t total) {
-    for (uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; g < total;
-         g += (uint64_t)gridDim.x * blockDim.x) {
-        const C v = in[g];
-        re[g] = (double)v.x;
-        im[g] = (double)v.y;
+// out = the state with its pending phases applied, canonical layout (nothing to move).
+template <typename C, int OUT, bool IN>
+__global__ void k_put(void* __restrict__ out, const C* __restrict__ in, uint64_t total, FastDiag p, int usep) {
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t g0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; g0 < total; g0 += PAIRS_PER_THREAD * stride) {
+        C v[PAIRS_PER_THREAD];
+#pragma unroll
+        for (int k = 0; k < PAIRS_PER_THREAD; ++k)
+            if (g0 + k * stride < total) v[k] = in[g0 + k * stride];
+#pragma unroll
+        for (int k = 0; k < PAIRS_PER_THREAD; ++k) {
+            const uint64_t g = g0 + k * stride;
+            if (g < total) put_out<OUT, C>(out, total, g, phased<IN>(p, usep, g, v[k]));
+        }
     }
 }
 
-template <typename C>
-__global__ void k_to_c128(double2* __restrict__ out, const C* __restrict__ in, uint64_t total) {
-    for (uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; g < total;
-         g += (uint64_t)gridDim.x * blockDim.x)
-        out[g] = make_double2((double)in[g].x, (double)in[g].y);
+// The same with fields moved and reflected.  Bound by HBM: one read and one write of
+// whole runs.  Gathering element by element wrote a swapped [14,14] complex64 state 16 KiB
+// apart and took 3.9 ms; through tiles (below) it takes 1.0.
+template <typename C, int OUT, bool IN>
+__global__ void __launch_bounds__(256) k_move(void* __restrict__ out, const C* __restrict__ in, uint64_t total,
+                                              MoveArgs a, FastDiag p, int usep) {
+    __shared__ double2 tile[(1 << MOVE_TILE_BITS) + (1 << (MOVE_TILE_BITS - 5))];
+    constexpr int PER = (1 << MOVE_TILE_BITS) / 256;
+    const int tid = threadIdx.x, n = 1 << a.nb;
+    uint64_t g0 = 0, mask = a.rest;
+    for (uint32_t b = blockIdx.x; mask && b; b >>= 1) {
+        const uint64_t low = mask & (~mask + 1ull);
+        if (b & 1u) g0 |= low;
+        mask &= mask - 1ull;
+    }
+    uint64_t c0 = a.flip;
+    for (int r = 0; r < a.nreg; ++r) c0 ^= ((g0 >> a.pshift[r]) & ((1ull << a.nq[r]) - 1ull)) << a.flw[r];
+    // bits of the tile's element tid + 256 k: those of tid once, those of k a register each
+    auto spread = [&](int e, const int* to) {
+        uint64_t v = 0;
+#pragma unroll
+        for (int i = 0; i < MOVE_TILE_BITS; ++i)
+            if (i < a.nb) v |= (uint64_t)((e >> i) & 1) << to[i];
+        return v;
+    };
+    const uint64_t p0 = g0 | spread(tid, a.pos);
+    C v[PER];
+#pragma unroll
+    for (int k = 0; k < PER; ++k)
+        if (tid + 256 * k < n) v[k] = in[p0 | spread(256 * k, a.pos)];
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+        const int e = tid + 256 * k;
+        if (e < n) tile[e + (e >> 5)] = phased<IN>(p, usep, p0 | spread(256 * k, a.pos), v[k]);
+    }
+    __syncthreads();
+    int ocp[MOVE_TILE_BITS];
+#pragma unroll
+    for (int i = 0; i < MOVE_TILE_BITS; ++i) ocp[i] = a.cpos[i];
+    const uint64_t c1 = c0 ^ spread(tid, ocp);
+    const int e1 = (int)spread(tid, a.ord);
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+        if (tid + 256 * k >= n) continue;
+        const int e = e1 | (int)spread(256 * k, a.ord);
+        put_out<OUT, C>(out, total, c1 ^ spread(256 * k, ocp), tile[e + (e >> 5)]);
+    }
 }
 
 template <typename C>
@@ -264,37 +310,87 @@ static unsigned grid_for(uint64_t total, unsigned block = 256) {
     return (unsigned)(b ? b : 1);
 }
 
+// Tile and permutation of the context's layout.
+static MoveArgs move_args(const CVDVContext* ctx) {
+    MoveArgs a{};
+    const int T = ctx->totalQbt;
+    int to[64];  // canonical position of every physical bit
+    a.nreg = ctx->numReg;
+    for (int r = 0; r < ctx->numReg; ++r) {
+        a.pshift[r] = ctx->pshift[r];
+        a.flw[r] = ctx->flw[r];
+        a.nq[r] = ctx->nq[r];
+        for (int b = 0; b < ctx->nq[r]; ++b) to[ctx->pshift[r] + b] = ctx->flw[r] + b;
+        if (ctx->refl[r]) a.flip |= ((1ull << ctx->nq[r]) - 1ull) << ctx->flw[r];
+    }
+    // half of the tile from the lowest physical bits, half from those that go lowest, the
+    // rest of its bits the next physical ones
+    const int nb = std::min(T, MOVE_TILE_BITS), half = std::min(T, MOVE_TILE_BITS / 2);
+    uint64_t in = 0;
+    for (int b = 0; b < T; ++b)
+        if (b < half || to[b] < half) in |= 1ull << b;
+    for (int b = 0; b < T && __builtin_popcountll(in) < nb; ++b) in |= 1ull << b;
+    a.rest = ((1ull << T) - 1ull) & ~in;
+    for (int b = 0; b < T; ++b)
+        if ((in >> b) & 1ull) a.pos[a.nb++] = b;
+    for (int i = 0; i < a.nb; ++i) a.ord[i] = i;
+    std::sort(a.ord, a.ord + a.nb, [&](int x, int y) { return to[a.pos[x]] < to[a.pos[y]]; });
+    for (int i = 0; i < a.nb; ++i) a.cpos[i] = to[a.pos[a.ord[i]]];
+    return a;
+}
+
+// dst = the context's state in canonical order with program p applied.
+template <int OUT>
+static void put_state(CVDVContext* ctx, void* dst, const DiagProg& p) {
+    const uint64_t n = ctx->totalSize;
+    const bool move = !ctx->canonical();
+    const MoveArgs a = move ? move_args(ctx) : MoveArgs{};
+    with_program(ctx, p, [&](auto in, const FastDiag& f, bool act, int per) {
+        constexpr bool IN = decltype(in)::value;
+        const int usep = act ? 1 : 0;
+        auto go = [&](auto* src) {
+            using C = std::remove_const_t<std::remove_pointer_t<decltype(src)>>;
+            if (move)
+                hipLaunchKernelGGL((k_move<C, OUT, IN>), dim3((unsigned)(n >> a.nb)), dim3(256), 0, ctx->stream, dst,
+                                   src, n, a, f, usep);
+            else
+                hipLaunchKernelGGL((k_put<C, OUT, IN>), dim3(grid_for((n + per - 1) / per)), dim3(256), 0,
+                                   ctx->stream, dst, src, n, f, usep);
+        };
+        if (ctx->prec == CVDV_C128) go((const double2*)ctx->state());
+        else go((const float2*)ctx->state());
+        HIPCHK(hipGetLastError());
+    });
+}
+
 void ctx_materialize(CVDVContext* ctx) {
     fft_settle(ctx);
     if (ctx->canonical()) {
         ctx_flush(ctx);
         return;
     }
-    LayoutArgs L{};
-    for (int r = 0; r < ctx->numReg; ++r) {
-        L.pshift[r] = ctx->pshift[r];
-        L.flw[r] = ctx->flw[r];
-        L.nq[r] = ctx->nq[r];
-        L.refl[r] = ctx->refl[r];
-    }
-    L.nreg = ctx->numReg;
-    DiagProg p = ctx_take_pending(ctx);
+    const DiagProg p = ctx_take_pending(ctx);
     void* dst = ctx->other();
-    const uint64_t n = ctx->totalSize;
     const int pid = prof_begin(ctx, KK_OTHER);
-    if (ctx->prec == CVDV_C128)
-        hipLaunchKernelGGL(k_materialize<double2>, dim3(grid_for(n)), dim3(256), 0, ctx->stream,
-                           (double2*)dst, (const double2*)ctx->state(), n, L, p);
-    else
-        hipLaunchKernelGGL(k_materialize<float2>, dim3(grid_for(n)), dim3(256), 0, ctx->stream,
-                           (float2*)dst, (const float2*)ctx->state(), n, L, p);
-    HIPCHK(hipGetLastError());
+    put_state<OUT_STATE>(ctx, dst, p);
     prof_end(ctx, pid);
     ctx->cur = 1 - ctx->cur;
     for (int r = 0; r < ctx->numReg; ++r) {
         ctx->pshift[r] = ctx->flw[r];
         ctx->refl[r] = 0;
     }
+}
+
+// The state for a readout, left as it is (phases pending, layout lazy): one pass, where
+// materialising it first takes two more.  A program that needs passes of its own is
+// applied to the state.
+template <int OUT>
+static void read_state(CVDVContext* ctx, void* dst) {
+    fft_settle(ctx);
+    FastDiag f;
+    bool act;
+    if (!inplace_diag(ctx, ctx->pending, f, act) && !diag_fits(ctx->pending, 0)) ctx_flush(ctx);
+    put_state<OUT>(ctx, dst, ctx->pending);
 }
 
 // ---------------------------------------------------------------- graph capture
@@ -597,16 +693,9 @@ void cvdvGetState(CVDVContext* ctx, double* realOut, double* imagOut) {
         return;
     }
     CVDV_TRY
-    ctx_materialize(ctx);
     const uint64_t n = ctx->totalSize;
     double* d = (double*)ctx_scratch(ctx, 2 * n * sizeof(double));
-    if (ctx->prec == CVDV_C128)
-        hipLaunchKernelGGL(k_split<double2>, dim3(grid_for(n)), dim3(256), 0, ctx->stream, d, d + n,
-                           (const double2*)ctx->state(), n);
-    else
-        hipLaunchKernelGGL(k_split<float2>, dim3(grid_for(n)), dim3(256), 0, ctx->stream, d, d + n,
-                           (const float2*)ctx->state(), n);
-    HIPCHK(hipGetLastError());
+    read_state<OUT_SPLIT>(ctx, d);
     HIPCHK(hipMemcpyAsync(realOut, d, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(hipMemcpyAsync(imagOut, d + n, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
@@ -712,16 +801,7 @@ void cvdvGetStateDevice(CVDVContext* ctx, void* d_dst) {
         return;
     }
     CVDV_TRY
-    ctx_materialize(ctx);
-    const uint64_t n = ctx->totalSize;
-    if (ctx->prec == CVDV_C128)
-        HIPCHK(hipMemcpyAsync(d_dst, ctx->state(), n * sizeof(double2), hipMemcpyDeviceToDevice,
-                              ctx->stream));
-    else {
-        hipLaunchKernelGGL(k_to_c128<float2>, dim3(grid_for(n)), dim3(256), 0, ctx->stream,
-                           (double2*)d_dst, (const float2*)ctx->state(), n);
-        HIPCHK(hipGetLastError());
-    }
+    read_state<OUT_C128>(ctx, d_dst);
     HIPCHK(hipStreamSynchronize(ctx->stream));
     CVDV_CATCH()
 }

@@ -26,6 +26,8 @@
 #include "cvdv_internal.h"
 #include "phase_eval.h"
 
+#include <type_traits>
+
 #define CVDV_FAST_TABS 6
 #define CVDV_FAST_GEN 4
 #define CVDV_TAB_SEL 4        // choice bits of one table
@@ -157,3 +159,22 @@ bool diag_fits(const DiagProg& p, uint64_t tileBits);
 
 // Largest table arena compile_diag can need for registers of at most maxNb qubits.
 size_t diag_arena_bound(int maxNb, size_t elemBytes);
+
+// The element-wise and pair kernels give each thread this many elements (pairs)
+// per iteration, their loads issued together.
+#define PAIRS_PER_THREAD 4
+
+// A kernel over the pairs (or elements) of the state with the program p applied: go(IN,
+// program, active, pairs a thread).  Evaluated in place one pair a thread is enough work,
+// and spreads small states over more of the chip.
+template <typename F>
+static void with_program(CVDVContext* ctx, const DiagProg& p, F go) {
+    FastDiag f;
+    bool act;
+    if (inplace_diag(ctx, p, f, act)) {
+        go(std::true_type{}, f, act, 1);
+    } else {
+        f = compile_diag(ctx, p, act);
+        go(std::false_type{}, f, act, PAIRS_PER_THREAD);
+    }
+}

@@ -11,7 +11,6 @@
 #include <cmath>
 #include <cstdio>
 #include <string>
-#include <type_traits>
 
 #include "cvdv_internal.h"
 #include "diag_fast.h"
@@ -21,9 +20,6 @@ static const double PI = 3.14159265358979323846;
 static const double SQRT2 = 1.41421356237309504880;
 
 // ---------------------------------------------------------------- kernels
-// The element-wise and pair kernels give each thread this many elements (pairs)
-// per iteration, their loads issued together.
-#define PAIRS_PER_THREAD 4
 
 // IN (here and below): the program is evaluated in place (inplace_diag).
 template <typename C, bool IN>
@@ -502,21 +498,6 @@ bool inplace_diag(const CVDVContext* ctx, const DiagProg& p, FastDiag& f, bool& 
     f.genrev = cvdv_frac(p.grev);
     active = f.ngen > 0 || f.genrev != 0.0;
     return true;
-}
-
-// A kernel over the pairs (or elements) of the state with the program p applied: go(IN,
-// program, active, pairs a thread).  Evaluated in place one pair a thread is enough work,
-// and spreads small states over more of the chip.
-template <typename F>
-static void with_program(CVDVContext* ctx, const DiagProg& p, F go) {
-    FastDiag f;
-    bool act;
-    if (inplace_diag(ctx, p, f, act)) {
-        go(std::true_type{}, f, act, 1);
-    } else {
-        f = compile_diag(ctx, p, act);
-        go(std::false_type{}, f, act, PAIRS_PER_THREAD);
-    }
 }
 
 // Bits of the flat index a term depends on.
