@@ -8,8 +8,13 @@
 #include <cmath>
 #include <cstdio>
 #include <algorithm>
+#include <atomic>
 #include <cstring>
+#include <mutex>
 #include <new>
+#include <exception>
+#include <thread>
+#include <vector>
 
 #include "cvdv_internal.h"
 #include "diag_fast.h"
@@ -73,6 +78,133 @@ void* ctx_scratch(CVDVContext* ctx, size_t bytes) {
         ctx->scratchBytes = bytes;
     }
     return ctx->scratch;
+}
+
+// ---------------------------------------------------------------- results to host memory
+// A result of some MiB lands in memory that the caller has just allocated: the runtime's
+// copy into pageable memory runs through one thread that takes a page fault for every
+// page it writes first (32 MiB: 3.2 ms, 0.6 of them the bus).  Here a few threads each
+// move chunks through pinned buffers of their own, so faults and copies overlap the bus
+// and each other: 32 MiB 1.26 ms, 8 MiB 0.64 -> 0.50, 4 MiB 0.33 -> 0.31, and no gain
+// below.  4 threads with 1 MiB chunks; 8 threads or 2 MiB chunks are as fast and pin
+// more, chunks of 512 KiB take 1.7 ms (a runtime call each).  The pinned buffers (8 MiB,
+// pinned within the first large copy, which is faster than the runtime's first one all
+// the same) are one set a process, used by one copy at a time (another thread's copy takes
+// the runtime's path meanwhile) and given back with the last context.
+#define HOST_COPY_THREADS 4
+#define HOST_COPY_SLOTS 2              // chunks in flight of a thread
+#define HOST_COPY_CHUNK (1u << 20)
+#define HOST_COPY_MIN (4u << 20)
+
+struct HostCopy {
+    std::mutex mu;   // held by the copy that uses the buffers
+    char* pinned = nullptr;
+    hipEvent_t ev[HOST_COPY_THREADS * HOST_COPY_SLOTS] = {};
+    int dev = -1;    // the events' device
+    std::mutex countMu;
+    int contexts = 0;
+
+    void release() {
+        for (hipEvent_t& e : ev) {
+            if (e) (void)hipEventDestroy(e);
+            e = nullptr;
+        }
+        if (pinned) (void)hipHostFree(pinned);
+        pinned = nullptr;
+        dev = -1;
+    }
+    bool prepare() {  // false: no pinned memory, the runtime's path serves
+        int d = 0;
+        if (hipGetDevice(&d) != hipSuccess) return false;
+        if (pinned && d == dev) return true;
+        release();
+        if (hipHostMalloc((void**)&pinned, (size_t)HOST_COPY_THREADS * HOST_COPY_SLOTS * HOST_COPY_CHUNK,
+                          hipHostMallocPortable) != hipSuccess) {
+            pinned = nullptr;
+            (void)hipGetLastError();
+            return false;
+        }
+        for (hipEvent_t& e : ev)
+            if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+                e = nullptr;
+                (void)hipGetLastError();
+                release();
+                return false;
+            }
+        dev = d;
+        return true;
+    }
+};
+static HostCopy& host_copy() {
+    static HostCopy* h = new HostCopy();  // never destroyed: contexts may outlive static destructors
+    return *h;
+}
+
+void host_copy_context(int delta) {
+    HostCopy& h = host_copy();
+    std::lock_guard<std::mutex> lk(h.countMu);
+    h.contexts += delta;
+    if (h.contexts == 0) {
+        std::lock_guard<std::mutex> use(h.mu);
+        h.release();
+    }
+}
+
+void copy_to_host(hipStream_t stream, void* dst, const void* src, size_t bytes) {
+    HostCopy& h = host_copy();
+    std::unique_lock<std::mutex> use(h.mu, std::defer_lock);
+    auto pageable = [&] {
+        hipPointerAttribute_t a;
+        if (hipPointerGetAttributes(&a, dst) == hipSuccess) return a.type == hipMemoryTypeUnregistered;
+        (void)hipGetLastError();
+        return true;
+    };
+    if (bytes < HOST_COPY_MIN || !pageable() || !use.try_lock() || !h.prepare()) {
+        HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream));
+        HIPCHK(hipStreamSynchronize(stream));
+        return;
+    }
+    const size_t chunks = (bytes + HOST_COPY_CHUNK - 1) / HOST_COPY_CHUNK;
+    const int nt = (int)std::min<size_t>(HOST_COPY_THREADS, chunks);
+    std::atomic<int> failed{0};
+    auto work = [&](int w) {
+        auto step = [&](hipError_t e) {
+            if (e != hipSuccess) failed.store((int)e);
+            return e == hipSuccess;
+        };
+        if (!step(hipSetDevice(h.dev))) return;
+        auto length = [&](size_t c) { return std::min((size_t)HOST_COPY_CHUNK, bytes - c * HOST_COPY_CHUNK); };
+        auto slot = [&](size_t i) { return w * HOST_COPY_SLOTS + (int)(i % HOST_COPY_SLOTS); };
+        auto fetch = [&](size_t i) {  // this thread's chunk number i
+            const size_t c = w + i * nt;
+            if (c >= chunks) return true;
+            return step(hipMemcpyAsync(h.pinned + (size_t)slot(i) * HOST_COPY_CHUNK,
+                                       (const char*)src + c * HOST_COPY_CHUNK, length(c), hipMemcpyDeviceToHost,
+                                       stream)) &&
+                   step(hipEventRecord(h.ev[slot(i)], stream));
+        };
+        for (size_t i = 0; i < HOST_COPY_SLOTS; ++i)
+            if (!fetch(i)) return;
+        for (size_t i = 0; w + i * nt < chunks; ++i) {
+            const size_t c = w + i * nt;
+            if (!step(hipEventSynchronize(h.ev[slot(i)]))) return;
+            std::memcpy((char*)dst + c * HOST_COPY_CHUNK, h.pinned + (size_t)slot(i) * HOST_COPY_CHUNK, length(c));
+            if (!fetch(i + HOST_COPY_SLOTS)) return;
+        }
+    };
+    std::vector<std::thread> th;
+    th.reserve(nt);
+    int started = 1;
+    try {
+        for (; started < nt; ++started) th.emplace_back(work, started);
+    } catch (const std::exception&) {
+    }
+    for (int w = started; w < nt; ++w) work(w);  // threads that could not start
+    work(0);
+    for (std::thread& t : th) t.join();
+    const hipError_t end = hipStreamSynchronize(stream);  // also what a failed worker left in flight
+    HIPCHK((hipError_t)failed.load());
+    HIPCHK(end);
 }
 
 // ---------------------------------------------------------------- profiling
@@ -249,8 +381,9 @@ __global__ void k_put(void* __restrict__ out, const C* __restrict__ in, uint64_t
 }
 
 // The same with fields moved and reflected.  Bound by HBM: one read and one write of
-// whole runs.  Gathering element by element wrote a swapped [14,14] complex64 state 16 KiB
-// apart and took 3.9 ms; through tiles (below) it takes 1.0.
+// whole runs.  Gathering element by element wrote a swapped [14,14] complex64 state 128 KiB
+// apart and took 3.9 ms, and widening it another 1.0; through tiles it is moved and
+// widened to complex128 (2 GiB read, 4 written) in 1.57.
 template <typename C, int OUT, bool IN>
 __global__ void __launch_bounds__(256) k_move(void* __restrict__ out, const C* __restrict__ in, uint64_t total,
                                               MoveArgs a, FastDiag p, int usep) {
@@ -463,6 +596,7 @@ static CVDVContext* create_impl(int numReg, const int* numQubits, int precision,
         return ctx;
     }
     HIPCHK(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
+    host_copy_context(1);
     return ctx;
 }
 
@@ -506,7 +640,10 @@ int cvdvGetPrecision(CVDVContext* ctx) { return ctx ? ctx->prec : -1; }
 void cvdvDestroy(CVDVContext* ctx) {
     if (!ctx || refuse_recording(ctx)) return;
     ctx_release(ctx);
-    if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
+    if (ctx->stream) {
+        (void)hipStreamDestroy(ctx->stream);
+        host_copy_context(-1);
+    }
     delete ctx;
 }
 
@@ -696,9 +833,8 @@ void cvdvGetState(CVDVContext* ctx, double* realOut, double* imagOut) {
     const uint64_t n = ctx->totalSize;
     double* d = (double*)ctx_scratch(ctx, 2 * n * sizeof(double));
     read_state<OUT_SPLIT>(ctx, d);
-    HIPCHK(hipMemcpyAsync(realOut, d, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipMemcpyAsync(imagOut, d + n, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
+    copy_to_host(ctx->stream, realOut, d, n * sizeof(double));
+    copy_to_host(ctx->stream, imagOut, d + n, n * sizeof(double));
     CVDV_CATCH()
 }
 

@@ -352,6 +352,10 @@ void fft_whole(CVDVContext* ctx, int sh, int nb, bool inverse, const DiagProg& p
 // measure.hip
 void marginal_probs(CVDVContext* ctx, const int* regs, int nsel, double* hostOut);
 
+// Copies device memory to (pageable) host memory behind the work on `stream` and waits
+// for it (ctx.hip).
+void copy_to_host(hipStream_t stream, void* dst, const void* src, size_t bytes);
+
 // scratch
 void* ctx_scratch(CVDVContext* ctx, size_t bytes);
 

@@ -233,8 +233,7 @@ static void marginal_core(CVDVContext* ctx, const int* regs, int nsel, double* h
         HIPCHK(hipGetLastError());
         res = fin;
     }
-    HIPCHK(hipMemcpyAsync(hostOut, res, outSize * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
+    copy_to_host(ctx->stream, hostOut, res, outSize * sizeof(double));
 }
 
 void marginal_probs(CVDVContext* ctx, const int* regs, int nsel, double* hostOut) {

@@ -416,8 +416,7 @@ static void get_wigner_grid(CVDVContext* ctx, int r, const double* xs, int nx, c
         dgemm_tn(ctx, c, np, K, dx / PI, (const double*)Ap, (uint64_t)c * K, (const double*)E, dout + x0, nx,
                  (uint64_t)np * nx, (int)outBlocks);
     }
-    HIPCHK(hipMemcpyAsync(out, dout, nZ * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
+    copy_to_host(ctx->stream, out, dout, nZ * sizeof(double));
 }
 
 static void get_husimi_grid(CVDVContext* ctx, int r, const double* qs, int nq, const double* ps, int np,
@@ -467,8 +466,7 @@ static void get_husimi_grid(CVDVContext* ctx, int r, const double* qs, int nq, c
     hipLaunchKernelGGL(k_grid_abs2, dim3(grid_for(nOut)), dim3(256), 0, ctx->stream, dout, H, S,
                        (uint64_t)np * nq, perSlice, dx / (PI * std::sqrt(PI)));
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(out, dout, nOut * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
+    copy_to_host(ctx->stream, out, dout, nOut * sizeof(double));
 }
 
 static bool grid_ok(CVDVContext* ctx, int r, const double* a, int na, const double* b, int nb, double* out) {

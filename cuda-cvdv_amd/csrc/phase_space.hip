@@ -527,8 +527,8 @@ static void wigner_device(CVDVContext* ctx, int r, void* dev, bool asComplex, do
 // The readouts below write their N x N result into `out`: host memory (through
 // a device scratch copy), or, with outOnDevice, caller device memory directly.
 static void finish_out(CVDVContext* ctx, double* out, const double* dev, uint64_t n, bool outOnDevice) {
-    if (!outOnDevice) HIPCHK(hipMemcpyAsync(out, dev, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
+    if (outOnDevice) HIPCHK(hipStreamSynchronize(ctx->stream));
+    else copy_to_host(ctx->stream, out, dev, n * sizeof(double));
 }
 
 static void get_wigner(CVDVContext* ctx, int r, double* out, bool outOnDevice) {
