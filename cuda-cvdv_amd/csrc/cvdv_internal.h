@@ -235,6 +235,7 @@ struct FtChainStep {
     DiagProg prog;
     int inverse;
     double scale;
+    int ctrl;  // >= 0: the direction is the other one where this index bit is set
 };
 struct FtChain {
     int open = 0;  // a gate is collecting
@@ -314,8 +315,12 @@ DiagProg ctx_take_pending(CVDVContext* ctx);
 void launch_diag(CVDVContext* ctx, const DiagProg& p);
 
 // fft.hip
+// ctrl >= 0 (only where fft_turns): the other direction where that index bit is set.
 void fft_register(CVDVContext* ctx, int pshift, int nbits, bool inverse, const DiagProg& pre,
-                  double outScale);
+                  double outScale, int ctrl = -1);
+// The field's transforms may take their direction from an index bit: each tile's pass
+// holds one value of it, or each thread's chain does.
+bool fft_turns(const CVDVContext* ctx, int sh, int nb, int ctrl);
 // largest dynamic LDS a workgroup may request on the current device
 size_t device_max_lds();
 void fft_generic_c128(CVDVContext* ctx, double2* data, double2* tmp, uint64_t total, int shift,
@@ -343,11 +348,11 @@ void fft_settle_bits(CVDVContext* ctx, uint64_t mask);
 // fft_chain.hip
 // A transform of field [sh, sh+nb) joins the current gate's chain (launched at once
 // outside a gate); false when it has to run by itself, nothing done.
-bool chain_accept(CVDVContext* ctx, int sh, int nb, bool inverse, const DiagProg& pre, double outScale);
+bool chain_accept(CVDVContext* ctx, int sh, int nb, bool inverse, const DiagProg& pre, double outScale, int ctrl);
 bool chain_field(const CVDVContext* ctx, int sh, int nb);  // its transforms run as chains
 void chain_flush(CVDVContext* ctx);                        // launch what was collected
 // fft.hip: a transform by itself (halves kept pending, or whole)
-void fft_whole(CVDVContext* ctx, int sh, int nb, bool inverse, const DiagProg& pre, double outScale);
+void fft_whole(CVDVContext* ctx, int sh, int nb, bool inverse, const DiagProg& pre, double outScale, int ctrl = -1);
 
 // measure.hip
 void marginal_probs(CVDVContext* ctx, const int* regs, int nsel, double* hostOut);

@@ -293,11 +293,17 @@ struct FftPass {
     int conjIn, conjOut;           // inverse = conj . forward . conj, split over the passes
     int conjLoad;                  // conjugate as loaded, before the four-step twiddle (the
                                    // second half of an inverse whose first half ran alone)
+    int conjCtl;                   // bit + 1: tiles with this index bit set run the other way
+                                   // (conjIn and conjOut flipped; the bit is the tile's); 0: none
     int lgInH1, lgInH2, lgInR;     // every stride is a power of two
     int lgOutH1, lgOutH2, lgOutR;
     double outScale;  // applied as exact v*hi + rounded v*lo (one FMA): an FP32 store stays unbiased
     int genSteps;     // 1: every generic term is affine in the tile's row index (the host checked)
 };
+
+__device__ __forceinline__ int tile_conj(const FftPass& d, int conj, uint64_t inBase) {
+    return d.conjCtl ? conj ^ (int)((inBase >> (d.conjCtl - 1)) & 1ull) : conj;
+}
 
 // The value lane `lane` of the wave holds (`lane` the same on every lane, and
 // that lane active).
@@ -710,11 +716,11 @@ __device__ __forceinline__ void stage0_pre(C* x, const FftPass& d, uint64_t inBa
                         x[k * RP + i] = cmul(x[k * RP + i], gen_factor<C>(P, pre, elem(k, i)));
             }
         }
-        if (d.conjIn) {
+        if (tile_conj(d, d.conjIn, inBase)) {
 #pragma unroll
             for (int i = 0; i < E; ++i) x[i].y = -x[i].y;
         }
-    } else if (d.conjIn) {
+    } else if (tile_conj(d, d.conjIn, inBase)) {
 #pragma unroll
         for (int i = 0; i < E; ++i) x[i].y = -x[i].y;
     }
@@ -724,7 +730,7 @@ __device__ __forceinline__ void stage0_pre(C* x, const FftPass& d, uint64_t inBa
 // elements before either store path.  Behind uniform branches: the compiler
 // would otherwise select per element and pay for the scale even when it is off.
 template <int E, typename R, typename C>
-__device__ __forceinline__ void out_finish(C* x, const FftPass& d, R scale, R scaleLo) {
+__device__ __forceinline__ void out_finish(C* x, const FftPass& d, int conj, R scale, R scaleLo) {
     if (d.useScale) {
 #pragma unroll
         for (int i = 0; i < E; ++i) {
@@ -732,7 +738,7 @@ __device__ __forceinline__ void out_finish(C* x, const FftPass& d, R scale, R sc
             x[i].y = fma(x[i].y, scale, x[i].y * scaleLo);
         }
     }
-    if (d.conjOut) {
+    if (conj) {
 #pragma unroll
         for (int i = 0; i < E; ++i) x[i].y = -x[i].y;
     }
@@ -885,10 +891,10 @@ k_fft_tile(const typename CT<R>::type* in, typename CT<R>::type* out, FftPass d,
         }
     };
     auto store = [&](C* x, uint64_t t, int ti) {
-        out_finish<E>(x, d, scale, scaleLo);
+        uint64_t lo0, inBase, outBase;
+        tile_base(t, lo0, inBase, outBase);
+        out_finish<E>(x, d, tile_conj(d, d.conjOut, inBase), scale, scaleLo);
         if (d.directOut) {
-            uint64_t lo0, inBase, outBase;
-            tile_base(t, lo0, inBase, outBase);
             last_store<RL, E, LGM, LGC>(out, x, d, outBase, scale, scaleLo, ti, nt);
             return;
         }
@@ -1046,7 +1052,7 @@ k_fft_fused(typename CT<R>::type* data, FftPass d, FftPass dD, FastDiag pre, int
     stage0_pre<R0, E, LGM, LGC, false, STG ? TM_STAGED : TM_ANY>(x, dD, natBase, P, pre, tw4, t2, nt, lds);
     stage_compute<R0, E, LGM, LGC, 0, false>(x, tw, t2, nt);
     run_stages<LGM, LGC, 1, E, false>(x, lds, tw, t2, nt);
-    out_finish<E>(x, d, scale, scaleLo);
+    out_finish<E>(x, d, d.conjOut, scale, scaleLo);
     last_store<RL, E, LGM, LGC>(data, x, d, base, scale, scaleLo, t2, nt);
 }
 
@@ -1333,11 +1339,13 @@ static FftCfg field_cfg(const CVDVContext* ctx, uint64_t total, int sh, int nb) 
     return it == ctx->fftCfg.end() ? FftCfg{} : it->second;
 }
 
-// Runs the FFT over field [sh, sh+nb) of a buffer of `total` elements.
+// Runs the FFT over field [sh, sh+nb) of a buffer of `total` elements, the other way
+// where the index bit `ctrl` (>= 0) is set (one-pass plans whose tiles hold one value of it).
 // Returns true when the result landed in the buffer returned by tmpFn.
 template <typename R, typename TmpFn>
 static bool fft_run(CVDVContext* ctx, typename CT<R>::type* data, TmpFn tmpFn, uint64_t total,
-                    int sh, int nb, bool inverse, const DiagProg& preProg, double outScale, int prec) {
+                    int sh, int nb, bool inverse, const DiagProg& preProg, double outScale, int prec,
+                    int ctrl = -1) {
     using C = typename CT<R>::type;
     const uint64_t N = 1ull << nb, S = 1ull << sh;
     const uint64_t H = total / (N * S);
@@ -1369,10 +1377,14 @@ static bool fft_run(CVDVContext* ctx, typename CT<R>::type* data, TmpFn tmpFn, u
         d.useScale = folded ? 0 : 1;
         d.conjIn = inv;
         d.conjOut = inv;
+        d.conjCtl = ctrl + 1;
         d.outScale = outScale;
+        if (ctrl >= 0 && ((tile_bits(d) >> ctrl) & 1ull))
+            throw CvdvError{CVDV_ERR_STATE, "transform direction by a bit that varies within a tile"};
         launch_pass<R>(ctx, data, data, d, pre, prec, 1);
         return false;
     }
+    if (ctrl >= 0) throw CvdvError{CVDV_ERR_STATE, "transform direction by a bit outside the one-pass plan"};
     if (total < 4096 || N <= 64) {
         // tiny state: direct DFT, out of place, FP64 accumulation rounded once
         // (per-element table reads: any choice bits)
@@ -1709,28 +1721,37 @@ void fft_prepare(CVDVContext* ctx) {
     }
 }
 
-void fft_register(CVDVContext* ctx, int pshift, int nbits, bool inverse, const DiagProg& pre,
-                  double outScale) {
-    if (chain_field(ctx, pshift, nbits)) {
-        if (FtDefer* rec = ctx->defer.find(pshift)) settle_one(ctx, *rec);
-        if (chain_accept(ctx, pshift, nbits, inverse, pre, outScale)) return;
-    }
-    chain_flush(ctx);
-    fft_whole(ctx, pshift, nbits, inverse, pre, outScale);
+bool fft_turns(const CVDVContext* ctx, int sh, int nb, int ctrl) {
+    if (ctx->rec || (ctrl >= sh && ctrl < sh + nb)) return false;
+    if (ctx->totalQbt <= FT_CHAIN_LG_SMALL) return chain_field(ctx, sh, nb);
+    const uint64_t N = 1ull << nb, S = 1ull << sh, total = ctx->totalSize;
+    const PassGeom g1{(int)N, S, total / (N * S), 1, 0, N * S, S, 0, N * S, S};
+    FftPass d{};
+    return fit_pass(g1, ctx->prec, d, true, field_cfg(ctx, total, sh, nb)) && !((tile_bits(d) >> ctrl) & 1ull);
 }
 
-void fft_whole(CVDVContext* ctx, int sh, int nb, bool inverse, const DiagProg& pre, double outScale) {
+void fft_register(CVDVContext* ctx, int pshift, int nbits, bool inverse, const DiagProg& pre,
+                  double outScale, int ctrl) {
+    if (chain_field(ctx, pshift, nbits)) {
+        if (FtDefer* rec = ctx->defer.find(pshift)) settle_one(ctx, *rec);
+        if (chain_accept(ctx, pshift, nbits, inverse, pre, outScale, ctrl)) return;
+    }
+    chain_flush(ctx);
+    fft_whole(ctx, pshift, nbits, inverse, pre, outScale, ctrl);
+}
+
+void fft_whole(CVDVContext* ctx, int sh, int nb, bool inverse, const DiagProg& pre, double outScale, int ctrl) {
     const bool done = ctx->prec == CVDV_C128 ? fft_deferred<double>(ctx, sh, nb, inverse, pre, outScale)
                                              : fft_deferred<float>(ctx, sh, nb, inverse, pre, outScale);
-    if (done) return;
+    if (done) return;  // (never with ctrl: a field with a one-pass plan keeps no half pending)
     if (FtDefer* rec = ctx->defer.find(sh)) settle_one(ctx, *rec);
     bool swapped;
     if (ctx->prec == CVDV_C128)
         swapped = fft_run<double>(ctx, (double2*)ctx->state(), [ctx] { return (double2*)ctx->other(); },
-                                  ctx->totalSize, sh, nb, inverse, pre, outScale, CVDV_C128);
+                                  ctx->totalSize, sh, nb, inverse, pre, outScale, CVDV_C128, ctrl);
     else
         swapped = fft_run<float>(ctx, (float2*)ctx->state(), [ctx] { return (float2*)ctx->other(); },
-                                 ctx->totalSize, sh, nb, inverse, pre, outScale, CVDV_MIXED);
+                                 ctx->totalSize, sh, nb, inverse, pre, outScale, CVDV_MIXED, ctrl);
     if (swapped) ctx->cur = 1 - ctx->cur;
 }
 

@@ -29,6 +29,7 @@
 // outside it; the rest vary over the rows in some other way.
 struct ChainStep {
     int inv, n, nrow;
+    int ctl;        // bit + 1: elements with this index bit set are transformed the other way; 0: none
     int byRow;      // every term has one value per row of a tile
     double grev, scale;
     DiagTerm t[FT_CHAIN_TERMS];
@@ -164,7 +165,9 @@ k_fft_chain(ChainArgs a, typename CT<R>::type* data, const typename CT<R>::type*
 #pragma unroll 1
     for (int s = 0; s < a.m; ++s) {
         const ChainStep& st = steps[s];
-        const int inv = __builtin_amdgcn_readfirstlane(st.inv);
+        const int ctl = __builtin_amdgcn_readfirstlane(st.ctl);
+        int inv = __builtin_amdgcn_readfirstlane(st.inv);
+        if (ctl) inv ^= (int)(own >> (ctl - 1)) & 1;
         // an opaque copy of the thread id: index math and twiddles, the same for every
         // step, would otherwise all be held across the steps
         int ti = tid;
@@ -307,7 +310,7 @@ void chain_flush(CVDVContext* ctx) {
     ch.n = 0;  // launched or, on an error, dropped
     if (m == 1 && ctx->totalQbt > FT_CHAIN_LG_SMALL) {
         const FtChainStep c = ch.st[0];
-        fft_whole(ctx, sh, nb, c.inverse != 0, c.prog, c.scale);
+        fft_whole(ctx, sh, nb, c.inverse != 0, c.prog, c.scale, c.ctrl);
         return;
     }
     int lgC, lgHb;
@@ -324,6 +327,7 @@ void chain_flush(CVDVContext* ctx) {
         const FtChainStep& c = ch.st[i];
         ChainStep& s = a.s[i];
         s.inv = c.inverse;
+        s.ctl = c.ctrl + 1;
         s.grev = cvdv_frac(c.prog.grev);
         s.scale = c.scale;
         s.byRow = 1;
@@ -358,7 +362,8 @@ bool chain_field(const CVDVContext* ctx, int sh, int nb) {
     return chain_tile(ctx, sh, nb, lgC, lgHb);
 }
 
-bool chain_accept(CVDVContext* ctx, int sh, int nb, bool inverse, const DiagProg& pre, double outScale) {
+bool chain_accept(CVDVContext* ctx, int sh, int nb, bool inverse, const DiagProg& pre, double outScale,
+                  int ctrl) {
     FtChain& ch = ctx->chain;
     const bool one = !ch.open || !ctx->fuseFt;
     if ((one && ctx->totalQbt > FT_CHAIN_LG_SMALL) || !chain_field(ctx, sh, nb)) return false;
@@ -368,7 +373,7 @@ bool chain_accept(CVDVContext* ctx, int sh, int nb, bool inverse, const DiagProg
     if (ch.n > 0 && (ch.sh != sh || ch.nb != nb || ch.n == FT_CHAIN_MAX)) chain_flush(ctx);
     ch.sh = sh;
     ch.nb = nb;
-    ch.st[ch.n++] = FtChainStep{pre, inverse ? 1 : 0, outScale};
+    ch.st[ch.n++] = FtChainStep{pre, inverse ? 1 : 0, outScale, ctrl};
     if (one) chain_flush(ctx);
     return true;
 }
