@@ -239,7 +239,7 @@ def run_c4(prec, circuits, n_seq, steps):
 # Sources each counter summary's kernels are compiled from (the phase programs
 # they apply come from gates.hip).  A summary records their fingerprint; a figure
 # is read from it only while the sources still match.
-FFT_SOURCES = ["fft.hip", "fft_bfly.h", "fft_stages.h", "diag_fast.h", "cvdv_internal.h", "gates.hip"]
+FFT_SOURCES = ["fft.hip", "fft_bfly.h", "fft_stages.h", "fft_pass.h", "fft_row.hip", "fft_row.h", "diag_fast.h", "cvdv_internal.h", "gates.hip"]
 BATCH_SOURCES = ["batch.hip", "fft_bfly.h", "diag_fast.h", "cvdv_internal.h", "gates.hip"]
 
 
@@ -1078,8 +1078,9 @@ def pmc_traffic(kind):
 
 # FFT pass kinds of the profile (cvdvProfileRead) -> kernel name and the register
 # transforms one launch performs (a fused pass completes one transform and starts
-# the next: one transform's worth; a lone half: half of one; a one-row tile: one)
-FFT_KINDS = {"fft_fused": ("k_fft_fused", 1.0), "fft_row": ("k_fft_tile (one-row)", 1.0),
+# the next: one transform's worth; a lone half: half of one; a row pass, which reads and
+# writes the state once for all the transforms that it chains: counted as one)
+FFT_KINDS = {"fft_fused": ("k_fft_fused", 1.0), "fft_row": ("k_fft_row", 1.0),
              "fft_half": ("k_fft_tile (four-step half)", 0.5)}
 
 

@@ -323,6 +323,7 @@ void fft_register(CVDVContext* ctx, int pshift, int nbits, bool inverse, const D
 bool fft_turns(const CVDVContext* ctx, int sh, int nb, int ctrl);
 // largest dynamic LDS a workgroup may request on the current device
 size_t device_max_lds();
+int device_cus();
 void fft_generic_c128(CVDVContext* ctx, double2* data, double2* tmp, uint64_t total, int shift,
                       int nbits, bool inverse, double outScale);
 void twiddle_cache_free(TwiddleCache* tc);
@@ -351,6 +352,11 @@ void fft_settle_bits(CVDVContext* ctx, uint64_t mask);
 bool chain_accept(CVDVContext* ctx, int sh, int nb, bool inverse, const DiagProg& pre, double outScale, int ctrl);
 bool chain_field(const CVDVContext* ctx, int sh, int nb);  // its transforms run as chains
 void chain_flush(CVDVContext* ctx);                        // launch what was collected
+// Contiguous complex64 rows of 2^13 and 2^14 points (fft_row.hip): fields whose transforms
+// the row kernel chains, the programs it takes, and one launch of a chain.
+bool row_field(const CVDVContext* ctx, int sh, int nb);
+bool row_accepts(int nb, const DiagProg& p);
+void fft_row_chain(CVDVContext* ctx, int nb, const FtChainStep* st, int m);
 // fft.hip: a transform by itself (halves kept pending, or whole)
 void fft_whole(CVDVContext* ctx, int sh, int nb, bool inverse, const DiagProg& pre, double outScale, int ctrl = -1);
 

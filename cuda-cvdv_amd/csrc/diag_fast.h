@@ -144,8 +144,11 @@ bool inplace_diag(const CVDVContext* ctx, const DiagProg& p, FastDiag& f, bool& 
 // tileBits: index bits that vary within one tile of a consumer that reads its
 // tables through a per-tile base; no choice bit is placed on them, so such a
 // consumer computes the choice once per tile.
+// first, *end: arena entries from and up to which the tables lie (a launch with several
+// programs keeps their tables side by side; the caller reserves the arena).
 FastDiag compile_diag(CVDVContext* ctx, const DiagProg& p, bool& active, double scale = 1.0,
-                      bool* scaleFolded = nullptr, uint64_t tileBits = 0);
+                      bool* scaleFolded = nullptr, uint64_t tileBits = 0, uint32_t first = 0,
+                      uint32_t* end = nullptr);
 
 // p with its linear polynomial terms over exactly the field [sh, sh + nb)
 // (control bit outside it) marked DT_LINF, as many as the generic-term slots

@@ -10,7 +10,7 @@
 //   * one HBM pass when the tile fits in LDS: C*M elements with C = 32 (c64)
 //     or 16 (c128) columns (256 bytes per row) for a strided register, or a
 //     whole contiguous register of up to 2^14 (c64) / 2^13 (c128) points in one
-//     workgroup (persistent and prefetching for c64 rows of 2^13 and 2^14);
+//     workgroup (c64 rows of 2^13 and 2^14: fft_row.hip);
 //   * otherwise the four-step split N = N1 * N2 (j = j1 + N1 j2):
 //       pass 1 (in place):  FFT over j2;
 //       pass 2 (out of place, transposing): times W_N^{j1 k2} on load, FFT
@@ -27,9 +27,8 @@
 #include <vector>
 
 #include "cvdv_internal.h"
-#include "diag_fast.h"
-#include "fft_bfly.h"
-#include "fft_stages.h"
+#include "fft_pass.h"
+#include "fft_row.h"
 
 static const long double PI_L = 3.141592653589793238462643383279502884L;
 
@@ -192,51 +191,36 @@ const void* fft_stage_table(TwiddleCache*& tcp, int logM, int prec) {
     return d;
 }
 
-// Split twiddles for the one-row tiles, which keep all twiddles in LDS.  Stage s
-// (radix R, sub-length L): L <= 64 stores W_{RL}^{p i} directly (p < L); larger L
-// stores W_{RL/64}^{a i} (a < L/64) and W_{RL}^{b i} (b < 64), and
-// W_{RL}^{p i} = W_{RL/64}^{(p>>6) i} W_{RL}^{(p&63) i}.  Layout per stage: the
-// direct segment, or the a segment then the b segment, each i-major (p fastest,
-// so the lanes of a wave read consecutive LDS words).
-static void split_values(int logM, std::vector<double>& re, std::vector<double>& im, std::vector<size_t>& segs) {
-    const StagePlan p = stage_plan(logM);
-    re.clear();
-    im.clear();
-    segs.clear();
-    auto put = [&](uint64_t e, uint64_t M) {
+// Twiddles of the row kernel (fft_row.hip): W_1024^{j p} of the middle stage (p < 32), then
+// W_M^{j t}, t < M/32, of the last as W_{M/32}^{j a} W_M^{j b}, t = 32 a + b; j-major.
+static void row_values(int lgm, std::vector<double>& re, std::vector<double>& im, std::vector<size_t>& segs) {
+    const uint64_t M = 1ull << lgm, RL = M >> 10;
+    auto put = [&](uint64_t e, uint64_t N) {
         double c, s;
-        host_twiddle(e, M, c, s);
+        host_twiddle(e, N, c, s);
         re.push_back(c);
         im.push_back(s);
     };
-    for (int st = 1; st < p.nst; ++st) {
-        const uint64_t R = (uint64_t)p.rad[st], L = (uint64_t)p.L[st], RL = R * L;
-        if (L <= 64) {
-            segs.push_back(re.size());
-            for (uint64_t i = 1; i < R; ++i)
-                for (uint64_t j = 0; j < L; ++j) put(i * j, RL);
-        } else {
-            segs.push_back(re.size());
-            for (uint64_t i = 1; i < R; ++i)
-                for (uint64_t a = 0; a < L / 64; ++a) put(i * a, RL / 64);
-            segs.push_back(re.size());
-            for (uint64_t i = 1; i < R; ++i)
-                for (uint64_t b = 0; b < 64; ++b) put(i * b, RL);
-        }
-    }
-    if (!segs.empty() && segs[0] == 0) segs.erase(segs.begin());
+    for (uint64_t j = 1; j < 32; ++j)
+        for (uint64_t p = 0; p < 32; ++p) put(j * p, 1024);
+    segs.push_back(re.size());
+    for (uint64_t j = 1; j < RL; ++j)
+        for (uint64_t a = 0; a < RL; ++a) put(j * a, M / 32);
+    segs.push_back(re.size());
+    for (uint64_t j = 1; j < RL; ++j)
+        for (uint64_t b = 0; b < 32; ++b) put(j * b, M);
 }
 
-static const void* split_table(CVDVContext* ctx, int logM, int prec) {
+static const void* row_table(CVDVContext* ctx, int lgm) {
     TwiddleCache* tc = cache(ctx);
-    const TwKey key{logM + 1000, prec};
+    const TwKey key{lgm + 1000, CVDV_MIXED};
     auto it = tc->stage.find(key);
     if (it != tc->stage.end()) return it->second;
     if (ctx->capturing) throw CvdvError{CVDV_ERR_UNSUPPORTED, "FFT table not prepared before the graph capture"};
     std::vector<double> re, im;
     std::vector<size_t> segs;
-    split_values(logM, re, im, segs);
-    void* d = upload_table(re, im, prec, segs);
+    row_values(lgm, re, im, segs);
+    void* d = upload_table(re, im, CVDV_MIXED, segs);
     tc->stage[key] = d;
     return d;
 }
@@ -279,471 +263,6 @@ size_t device_max_lds() {
     return (size_t)v;
 }
 
-// ---------------------------------------------------------------- pass descriptor
-struct FftPass {
-    int lgM, lgC, lgHb;            // tile = [Hb][M][C] (lgM also selects the kernel instance)
-    int lgNLoBlk, lgNH2Blk;        // tiles = nH1 * nH2Blk * nLoBlk
-    uint64_t nTiles;
-    int rowFastOut;                // linear order of the staged store after the column index
-    int vecOut;                    // 1: pairs of complex64 stored as one 16-byte access
-    int directOut;                 // 1: last stage stores straight to global (coalesced rows)
-    int tw4, tw4Shift, tw4HiBits, tw4LogN;
-    int tw4Uni;                    // 1: the twiddle's second index is the same over the tile
-    int usePre, useScale;
-    int conjIn, conjOut;           // inverse = conj . forward . conj, split over the passes
-    int conjLoad;                  // conjugate as loaded, before the four-step twiddle (the
-                                   // second half of an inverse whose first half ran alone)
-    int conjCtl;                   // bit + 1: tiles with this index bit set run the other way
-                                   // (conjIn and conjOut flipped; the bit is the tile's); 0: none
-    int lgInH1, lgInH2, lgInR;     // every stride is a power of two
-    int lgOutH1, lgOutH2, lgOutR;
-    double outScale;  // applied as exact v*hi + rounded v*lo (one FMA): an FP32 store stays unbiased
-    int genSteps;     // 1: every generic term is affine in the tile's row index (the host checked)
-};
-
-__device__ __forceinline__ int tile_conj(const FftPass& d, int conj, uint64_t inBase) {
-    return d.conjCtl ? conj ^ (int)((inBase >> (d.conjCtl - 1)) & 1ull) : conj;
-}
-
-// The value lane `lane` of the wave holds (`lane` the same on every lane, and
-// that lane active).
-__device__ __forceinline__ float2 lane_value(float2 v, int lane) {
-    return make_float2(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(v.x), lane)),
-                       __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v.y), lane)));
-}
-__device__ __forceinline__ double2 lane_value(double2 v, int lane) {
-    auto rd = [lane](double d) {
-        const long long b = __double_as_longlong(d);
-        const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)b, lane);
-        const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(b >> 32), lane);
-        return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-    };
-    return make_double2(rd(v.x), rd(v.y));
-}
-
-// Tile element e (linear) -> (c, row, hb) in the given order.
-template <int LGM>
-__device__ __forceinline__ void tile_coords(int e, int lgC, int lgHb, int rowFast, int& c, int& row, int& hb) {
-    c = e & ((1 << lgC) - 1);
-    const int rest = e >> lgC;
-    const int lgLo = rowFast ? LGM : lgHb;  // selects, not branches on references (no scratch)
-    const int lo = rest & ((1 << lgLo) - 1), hi = rest >> lgLo;
-    row = rowFast ? lo : hi;
-    hb = rowFast ? hi : lo;
-}
-
-// The compiled pending program, staged in LDS so its runtime-length loops read
-// LDS instead of forcing a scratch copy of the kernel argument.
-struct PreLds {
-    DiagTab tab[CVDV_FAST_TABS];
-    DiagTerm gen[CVDV_FAST_GEN];
-};
-
-// The generic terms over a one-row tile (only the transformed field
-// [fs, fs + fn) varies inside it): when every term is affine in that field's
-// coordinate m, their sum is a·m + b (mod 1) with per-tile a, b, and one FP64
-// fma per element replaces the per-term evaluation.  a is reduced mod 1 (m is
-// an integer), so a·m stays below 2^(fn-1) and keeps ~2^-40 absolute accuracy.
-struct GenFold {
-    double a, b;
-    int ok;
-};
-
-__device__ __forceinline__ bool field_overlaps(int sh, int nb, int fs, int fn) {
-    return sh < fs + fn && fs < sh + nb;
-}
-
-__device__ __forceinline__ GenFold fold_generic(const PreLds& P, const FastDiag& pre, uint64_t g0, int fs, int fn) {
-    GenFold f{0.0, pre.genrev, 1};
-    for (int i = 0; i < pre.ngen; ++i) {
-        const DiagTerm& T = P.gen[i];
-        if (T.ctrl >= 0 && T.ctrl >= fs && T.ctrl < fs + fn) f.ok = 0;
-        const double sg = (T.ctrl >= 0 && ((g0 >> T.ctrl) & 1ull)) ? -1.0 : 1.0;
-        const bool in1 = T.sh1 == fs && T.nb1 == fn;
-        if (T.kind == DT_BILIN) {
-            const bool in2 = T.sh2 == fs && T.nb2 == fn;
-            if ((!in1 && field_overlaps(T.sh1, T.nb1, fs, fn)) || (!in2 && field_overlaps(T.sh2, T.nb2, fs, fn)) ||
-                (in1 && in2))
-                f.ok = 0;
-            else if (in1)
-                f.a += cvdv_frac(sg * T.c1 * diag_field_m(g0, T.sh2, T.nb2));
-            else if (in2)
-                f.a += cvdv_frac(sg * T.c1 * diag_field_m(g0, T.sh1, T.nb1));
-            else
-                f.b += cvdv_frac(sg * diag_term_rev(T, g0));
-        } else if (T.kind == DT_POLY || T.kind == DT_LINF) {
-            if (in1 && T.c2 == 0.0 && T.c3 == 0.0)
-                f.a += cvdv_frac(sg * T.c1);
-            else if (field_overlaps(T.sh1, T.nb1, fs, fn))
-                f.ok = 0;
-            else
-                f.b += cvdv_frac(sg * diag_term_rev(T, g0));
-        } else {
-            if (T.sh1 >= fs && T.sh1 < fs + fn) f.ok = 0;
-            else f.b += cvdv_frac(sg * diag_term_rev(T, g0));
-        }
-    }
-    f.a = cvdv_frac(f.a);
-    f.b = cvdv_frac(f.b);
-    return f;
-}
-
-// Phase of the generic (untabulated) terms at element g.
-template <typename C>
-__device__ __forceinline__ C gen_factor(const PreLds& P, const FastDiag& pre, uint64_t g) {
-    using R = decltype(C{}.x);
-    double r = pre.genrev;
-    for (int i = 0; i < pre.ngen; ++i) r += cvdv_frac(diag_term_rev(P.gen[i], g));
-    return unit_rev_fast(cvdv_frac(r), R(0));
-}
-
-// Stage-0 inputs straight from global memory (issued early: a tile ahead).
-template <int RP, int E, int LGM, int LGC, typename C>
-__device__ __forceinline__ void stage0_load(const C* __restrict__ in, C* x, const FftPass& d, uint64_t inBase,
-                                            int tid, int nt) {
-    constexpr int NB = E / RP;
-    constexpr int LGR = RP == 8 ? 3 : (RP == 4 ? 2 : 1);
-    constexpr int lgMq = LGM - LGR;
-#pragma unroll
-    for (int k = 0; k < NB; ++k) {
-        const BflyPos p = bfly_pos<RP, LGM, E>(tid, k, nt, LGC);
-        const uint64_t g0 = inBase + ((uint64_t)p.hb << d.lgInH2) + ((uint64_t)p.q << d.lgInR) + p.c;
-#pragma unroll
-        for (int i = 0; i < RP; ++i) x[k * RP + i] = in[g0 + ((uint64_t)(i << lgMq) << d.lgInR)];
-    }
-}
-
-// Pending phases, the four-step twiddle W_N^{j1 k2} of a second pass (row j1 =
-// the transformed index, k2 = (g >> tw4Shift) mod 2^tw4HiBits; TW4: the
-// instance may carry one) and the input conjugation of an inverse on the loaded
-// inputs.  TM, how the phase tables are read:
-//   TM_ROWS   every table is read by row (the host checked, table_by_row()), one
-//             load per element at a row offset (one-row tiles);
-//   TM_ANY    tables of several columns stage their product by row in LDS when
-//             every table allows it, else each element takes its flat index;
-//   TM_STAGED every table is read by row (the host checked, tile_tables_by_row())
-//             and is staged by row; generic terms go through the free exchange
-//             buffer (complex64: their row steps per column and row block;
-//             complex128: each element's factor from a rolled loop), which
-//             keeps their FP64 temporaries off the other elements' registers.
-// TM_NONE: the pass applies no phases (only the four-step twiddle, if TW4).
-enum { TM_ROWS = 0, TM_ANY = 1, TM_STAGED = 2, TM_NONE = 3 };
-template <int RP, int E, int LGM, int LGC, bool TW4, int TM, typename C>
-__device__ __forceinline__ void stage0_pre(C* x, const FftPass& d, uint64_t inBase, const PreLds& P,
-                                           const FastDiag& pre, const C* __restrict__ tw4, int tid, int nt,
-                                           C* sRow) {
-    constexpr int NB = E / RP;
-    constexpr int LGR = RP == 8 ? 3 : (RP == 4 ? 2 : 1);
-    constexpr int lgMq = LGM - LGR;
-    if (TW4 && d.tw4) {
-        // second four-step pass: straight-line, so these loads issue with the
-        // tile's input loads and share their wait
-        if (d.tw4Uni) {
-            // k2 is the tile's (no tile index bit selects it), so W^{k2 (q + i M/RP)} =
-            // W^{k2 q} W^{k2 i M/RP} takes one gathered and RP-1 tile-uniform
-            // (scalar) loads per butterfly instead of RP gathers
-            const uint32_t nmask = (1u << d.tw4LogN) - 1u;
-            const uint32_t k2 = (uint32_t)(inBase >> d.tw4Shift) & ((1u << d.tw4HiBits) - 1u);
-            C st[RP];
-#pragma unroll
-            for (int i = 1; i < RP; ++i) st[i] = tw4[(k2 * (uint32_t)(i << lgMq)) & nmask];
-#pragma unroll
-            for (int k = 0; k < NB; ++k) {
-                const BflyPos p = bfly_pos<RP, LGM, E>(tid, k, nt, LGC);
-                const C b = tw4[(k2 * (uint32_t)p.q) & nmask];
-                x[k * RP] = cmul(x[k * RP], b);
-#pragma unroll
-                for (int i = 1; i < RP; ++i) x[k * RP + i] = cmul(x[k * RP + i], cmul(b, st[i]));
-            }
-        } else {
-            // k2 differs within the tile (between row blocks or columns): per
-            // butterfly, gather W^{k2 q} and
-            // w = W^{k2 M/RP}; the powers w^i come from a multiplication tree of
-            // depth log2(RP)
-#pragma unroll
-            for (int k = 0; k < NB; ++k) {
-                const BflyPos p = bfly_pos<RP, LGM, E>(tid, k, nt, LGC);
-                const uint64_t g0 = inBase + ((uint64_t)p.hb << d.lgInH2) + ((uint64_t)p.q << d.lgInR) + p.c;
-                const uint32_t nmask = (1u << d.tw4LogN) - 1u;
-                const uint32_t k2 = (uint32_t)(g0 >> d.tw4Shift) & ((1u << d.tw4HiBits) - 1u);
-                const C b = tw4[(k2 * (uint32_t)p.q) & nmask];
-                C st[RP];
-                st[1] = tw4[(k2 << lgMq) & nmask];
-#pragma unroll
-                for (int i = 2; i < RP; ++i) st[i] = cmul(st[i / 2], st[i - i / 2]);
-                x[k * RP] = cmul(x[k * RP], b);
-#pragma unroll
-                for (int i = 1; i < RP; ++i) x[k * RP + i] = cmul(x[k * RP + i], cmul(b, st[i]));
-            }
-        }
-    }
-    if (TM != TM_NONE && d.usePre) {
-        int tt = tid;
-        auto elem = [&](int k, int i) {
-            const BflyPos p = bfly_pos<RP, LGM, E>(tt, k, nt, LGC);
-            return inBase + ((uint64_t)p.hb << d.lgInH2) + ((uint64_t)p.q << d.lgInR) + p.c +
-                   ((uint64_t)(i << lgMq) << d.lgInR);
-        };
-        // Table-major: the E entries of one table are loaded together, so a wave
-        // has E loads in flight instead of one dependent load per element.  The
-        // first table is applied in straight-line code, so its loads issue with
-        // the tile's input loads and share their wait (a loop that touches x
-        // would wait for x's loads before issuing its first table load).
-        // A table whose field misses the tile's column and row-block bits, and
-        // holds all or none of its row bits, is read at base + (row << s) with a
-        // per-tile base and conjugation: 32-bit indices instead of each element's
-        // 64-bit flat index.
-        const int rowLo = d.lgInR, rowHi = d.lgInR + LGM;
-        auto hits = [](int sh, int nb, int lo, int n) { return n > 0 && sh < lo + n && lo < sh + nb; };
-        // Where a table is read through the tile's base: the base, the row shift
-        // (31: the row does not index it) and the conjugation.
-        struct TabAt {
-            DiagTab T;
-            bool fast, cj;
-            int s;
-            const C* tb;
-        };
-        auto tab_at = [&](const DiagTab& TL) {
-            TabAt A;
-            // the descriptor is read from LDS into vector registers; it is the
-            // same for every lane, so keep it in scalar registers
-            DiagTab& T = A.T;
-            T.sh = __builtin_amdgcn_readfirstlane(TL.sh);
-            T.nb = __builtin_amdgcn_readfirstlane(TL.nb);
-            T.ctrl = __builtin_amdgcn_readfirstlane(TL.ctrl);
-            T.off = (uint32_t)__builtin_amdgcn_readfirstlane((int)TL.off);
-            T.nsel = __builtin_amdgcn_readfirstlane(TL.nsel);
-            T.sel = (uint32_t)__builtin_amdgcn_readfirstlane((int)TL.sel);
-            const bool rowIn = T.sh <= rowLo && rowHi <= T.sh + T.nb;
-            auto varies = [&](int b) {
-                return b >= 0 && (b < LGC || (b >= rowLo && b < rowHi) ||
-                                  (d.lgHb > 0 && b >= d.lgInH2 && b < d.lgInH2 + d.lgHb));
-            };
-            bool ctrlVar = varies(T.ctrl);
-#pragma unroll
-            for (int j = 0; j < CVDV_TAB_SEL; ++j)
-                if (j < T.nsel) ctrlVar = ctrlVar || varies(tab_sel(T, j));
-            A.fast = !hits(T.sh, T.nb, 0, LGC) && !hits(T.sh, T.nb, d.lgInH2, d.lgHb) &&
-                     (rowIn || !hits(T.sh, T.nb, rowLo, LGM)) && !ctrlVar;
-            // choice bits are tile-uniform here: they only move the tile's base
-            A.tb = (const C*)pre.arena + T.off + (uint32_t)((inBase >> T.sh) & ((1ull << T.nb) - 1ull)) +
-                   (T.nsel > 0 ? tab_choice(T, inBase) : 0u);
-            A.s = rowIn ? rowLo - T.sh : 31;
-            A.cj = T.ctrl >= 0 && ((inBase >> T.ctrl) & 1ull);
-            return A;
-        };
-        auto apply_table = [&](const DiagTab& TL) {
-            const TabAt A = tab_at(TL);
-            const DiagTab& T = A.T;
-            const bool fast = A.fast;
-            constexpr int CH = sizeof(C) == 16 ? (RP < 8 ? 2 : 4) : 8;  // entries in flight per batch
-            if (TM == TM_ROWS || fast) {
-                const C* tb = A.tb;
-                const int s = A.s;
-                const bool cj = A.cj;
-#pragma unroll
-                for (int j0 = 0; j0 < E; j0 += CH) {
-                    C e[CH];
-#pragma unroll
-                    for (int j = 0; j < CH; ++j) {
-                        const BflyPos p = bfly_pos<RP, LGM, E>(tt, (j0 + j) / RP, nt, LGC);
-                        const uint32_t row = (uint32_t)(p.q + (((j0 + j) % RP) << lgMq));
-                        e[j] = tb[s < 31 ? (row << s) : 0u];
-                        if (cj) e[j].y = -e[j].y;
-                    }
-#pragma unroll
-                    for (int j = 0; j < CH; ++j) x[j0 + j] = cmul(x[j0 + j], e[j]);
-                }
-            } else if constexpr (TM == TM_ANY) {
-                // per element; the choice bits are tile-uniform (the tables were
-                // compiled for this tiling), so the choice is one per tile
-                const C* tb = (const C*)pre.arena + T.off + (T.nsel > 0 ? tab_choice(T, inBase) : 0u);
-#pragma unroll
-                for (int j0 = 0; j0 < E; j0 += CH) {
-                    C e[CH];
-#pragma unroll
-                    for (int j = 0; j < CH; ++j) {
-                        const uint64_t g = elem((j0 + j) / RP, (j0 + j) % RP);
-                        e[j] = tb[(uint32_t)((g >> T.sh) & ((1ull << T.nb) - 1ull))];
-                        if (T.ctrl >= 0 && ((g >> T.ctrl) & 1ull)) e[j].y = -e[j].y;
-                    }
-#pragma unroll
-                    for (int j = 0; j < CH; ++j) x[j0 + j] = cmul(x[j0 + j], e[j]);
-                }
-            }
-        };
-        // Generic terms affine in the row index (complex64 staged instances always;
-        // otherwise when d.genSteps): a butterfly's rows are q + i M/RP with its
-        // column and row block (position j) fixed, so its phases are P(q) + i D_j.
-        // The steps e^{2 pi i i D_j} go to the free exchange buffer, RP-1 per
-        // position, one sin/cos each; a butterfly then takes one FP64 evaluation,
-        // one sin/cos e0 and RP-1 products e0 * step.  The caller puts a barrier
-        // before the buffer is written again.
-        auto row_steps = [&]() {
-            using RR = decltype(C{}.x);
-            const int nj = (nt * E) >> LGM;
-#pragma unroll 1
-            for (int s = tt; s < nj * (RP - 1); s += nt) {
-                const int j = s / (RP - 1), i = s - j * (RP - 1) + 1;
-                const uint64_t g0 =
-                    inBase + ((uint64_t)(j >> LGC) << d.lgInH2) + (uint64_t)(j & ((1 << LGC) - 1));
-                const uint64_t g1 = g0 + ((uint64_t)(1 << lgMq) << d.lgInR);
-                double dl = 0.0;
-                for (int t = 0; t < pre.ngen; ++t)
-                    dl += cvdv_frac(diag_term_rev(P.gen[t], g1) - diag_term_rev(P.gen[t], g0));
-                sRow[s] = unit_rev_fast(cvdv_frac((double)i * cvdv_frac(dl)), RR(0));
-            }
-            lds_barrier();
-#pragma unroll
-            for (int k = 0; k < NB; ++k) {
-                const BflyPos p = bfly_pos<RP, LGM, E>(tt, k, nt, LGC);
-                const uint64_t g0 = elem(k, 0);
-                double p0 = pre.genrev;
-                for (int t = 0; t < pre.ngen; ++t) p0 += cvdv_frac(diag_term_rev(P.gen[t], g0));
-                const C e0 = unit_rev_fast(cvdv_frac(p0), RR(0));
-                const C* st = sRow + (p.c | (p.hb << LGC)) * (RP - 1) - 1;
-                x[k * RP] = cmul(x[k * RP], e0);
-#pragma unroll
-                for (int i = 1; i < RP; ++i) x[k * RP + i] = cmul(x[k * RP + i], cmul(e0, st[i]));
-            }
-        };
-        bool staged = false;
-        if constexpr (LGC > 0 && TM != TM_ROWS) {
-            // Tiles of several columns: when every table is read by row, their
-            // product over the tile's M rows is staged in LDS (one table load per
-            // row instead of one per element), and each element takes one LDS
-            // read and one product.  The exchange buffer is free before the
-            // stages; a barrier hands it back.
-            bool byRow = pre.ntab > 0;
-            if constexpr (TM == TM_ANY)
-                for (int t = 0; t < pre.ntab; ++t) byRow = byRow && tab_at(P.tab[t]).fast;
-            if (byRow) {
-                for (int r = tid; r < (1 << LGM); r += nt) {
-                    C f = cmk<C>(1.0, 0.0);
-                    for (int t = 0; t < pre.ntab; ++t) {
-                        const TabAt A = tab_at(P.tab[t]);
-                        C e = A.tb[A.s < 31 ? ((uint32_t)r << A.s) : 0u];
-                        if (A.cj) e.y = -e.y;
-                        f = t == 0 ? e : cmul(f, e);
-                    }
-                    sRow[r] = f;
-                }
-                lds_barrier();
-#pragma unroll
-                for (int k = 0; k < NB; ++k) {
-                    const BflyPos p = bfly_pos<RP, LGM, E>(tt, k, nt, LGC);
-#pragma unroll
-                    for (int i = 0; i < RP; ++i) x[k * RP + i] = cmul(x[k * RP + i], sRow[p.q + (i << lgMq)]);
-                }
-                lds_barrier();
-                staged = true;
-            }
-        }
-        if (TM != TM_STAGED && !staged) {
-            if (pre.ntab > 0) apply_table(P.tab[0]);
-            for (int t = 1; t < pre.ntab; ++t) {
-                // opaque: the element indices are recomputed per table, not held
-                asm volatile("" : "+v"(tt));
-                apply_table(P.tab[t]);
-            }
-        }
-        if constexpr (TM == TM_STAGED && LGC > 0) {
-            if (pre.ngen > 0) {
-                using RR = decltype(C{}.x);
-                if (sizeof(C) == 8 || d.genSteps) {
-                    row_steps();
-                } else {
-                    // complex128 with terms that are not affine in the rows: one
-                    // element per iteration, its terms evaluated exactly; its factor
-                    // goes to its own slot of the exchange buffer (element-major, so
-                    // a wave's writes are consecutive), then every element takes its
-                    // product.
-#pragma unroll 1
-                    for (int k = 0; k < NB; ++k) {
-#pragma unroll 1
-                        for (int i = 0; i < RP; ++i) {
-                            const uint64_t g = elem(k, i);
-                            double r = pre.genrev;
-                            for (int t = 0; t < pre.ngen; ++t) r += cvdv_frac(diag_term_rev(P.gen[t], g));
-                            sRow[(k * RP + i) * nt + tt] = unit_rev_fast(cvdv_frac(r), RR(0));
-                        }
-                    }
-#pragma unroll
-                    for (int j = 0; j < E; ++j) x[j] = cmul(x[j], sRow[j * nt + tt]);
-                }
-                lds_barrier();  // the stages that follow write other threads' slots
-            }
-        } else if (pre.ngen > 0) {
-            asm volatile("" : "+v"(tt));
-            // one-row tiles: the terms are affine in the row coordinate
-            GenFold gf{0.0, 0.0, 0};
-            if (LGC == 0 && d.lgHb == 0) gf = fold_generic(P, pre, inBase, d.lgInR, LGM);
-            if (gf.ok) {
-                using R = decltype(C{}.x);
-                // A butterfly's rows are q + i M/RP, so its phases are e^{2 pi i (a m0 + b)}
-                // times the tile-wide steps e^{2 pi i a 2 i M/RP}: one sin/cos per
-                // butterfly, and RP-1 per tile (uniform across the wave).
-                C st[RP];
-                if (nt >= 64) {
-                    // full waves: lane i evaluates step i, the others read it
-                    const int li = (int)__builtin_amdgcn_mbcnt_lo(~0u, 0u) & (RP - 1);
-                    const C mine = unit_rev_fast(cvdv_frac(gf.a * (double)(2 * (li << lgMq))), R(0));
-#pragma unroll
-                    for (int i = 1; i < RP; ++i) st[i] = lane_value(mine, i);
-                } else {
-#pragma unroll
-                    for (int i = 1; i < RP; ++i)
-                        st[i] = unit_rev_fast(cvdv_frac(gf.a * (double)(2 * (i << lgMq))), R(0));
-                }
-#pragma unroll
-                for (int k = 0; k < NB; ++k) {
-                    const BflyPos p = bfly_pos<RP, LGM, E>(tt, k, nt, LGC);
-                    const double m0 = (double)(2 * p.q + 1 - (1 << LGM));
-                    const C e0 = unit_rev_fast(cvdv_frac(fma(gf.a, m0, gf.b)), R(0));
-                    x[k * RP] = cmul(x[k * RP], e0);
-#pragma unroll
-                    for (int i = 1; i < RP; ++i) x[k * RP + i] = cmul(x[k * RP + i], cmul(e0, st[i]));
-                }
-            } else if (TM != TM_ROWS && d.genSteps) {
-                // tiles of several columns or row blocks
-                row_steps();
-                lds_barrier();  // the stages that follow write the exchange buffer
-            } else {
-#pragma unroll
-                for (int k = 0; k < NB; ++k)
-#pragma unroll
-                    for (int i = 0; i < RP; ++i)
-                        x[k * RP + i] = cmul(x[k * RP + i], gen_factor<C>(P, pre, elem(k, i)));
-            }
-        }
-        if (tile_conj(d, d.conjIn, inBase)) {
-#pragma unroll
-            for (int i = 0; i < E; ++i) x[i].y = -x[i].y;
-        }
-    } else if (tile_conj(d, d.conjIn, inBase)) {
-#pragma unroll
-        for (int i = 0; i < E; ++i) x[i].y = -x[i].y;
-    }
-}
-
-// Output scale and conjugation (inverse), applied to a thread's transformed
-// elements before either store path.  Behind uniform branches: the compiler
-// would otherwise select per element and pay for the scale even when it is off.
-template <int E, typename R, typename C>
-__device__ __forceinline__ void out_finish(C* x, const FftPass& d, int conj, R scale, R scaleLo) {
-    if (d.useScale) {
-#pragma unroll
-        for (int i = 0; i < E; ++i) {
-            x[i].x = fma(x[i].x, scale, x[i].x * scaleLo);
-            x[i].y = fma(x[i].y, scale, x[i].y * scaleLo);
-        }
-    }
-    if (conj) {
-#pragma unroll
-        for (int i = 0; i < E; ++i) x[i].y = -x[i].y;
-    }
-}
-
 // Last-stage outputs straight to global memory (rows q + m*M/RP of column c).
 template <int RP, int E, int LGM, int LGC, typename R, typename C>
 __device__ __forceinline__ void last_store(C* __restrict__ out, const C* v, const FftPass& d, uint64_t outBase,
@@ -770,7 +289,6 @@ constexpr bool one_row_layouts() {
     return sizeof(R) == 4 && LGC == 0 && LGM >= 13 && Plan<LGM>::lgr(0) == 3 && Plan<LGM>::lgr(1) == 3;
 }
 
-// PF: persistent workgroups that prefetch the next tile (one-row tiles).
 // Workgroup size bound: one-row tiles of 2^12 points and more take up to 1024
 // threads; every other tile fits 64 KiB of LDS, i.e. at most 512 (complex64) or
 // 256 (complex128) threads at 8 elements each.
@@ -779,7 +297,7 @@ constexpr int tile_threads_max() {
     return (LGC == 0 && LGM >= 12) ? 1024 : (sizeof(R) == 4 ? 512 : 256);
 }
 
-template <typename R, int LGM, int LGC, int E, bool PF>
+template <typename R, int LGM, int LGC, int E>
 __global__ void __launch_bounds__((tile_threads_max<R, LGM, LGC>()))
 k_fft_tile(const typename CT<R>::type* in, typename CT<R>::type* out, FftPass d, FastDiag pre,
            const typename CT<R>::type* __restrict__ tw, const typename CT<R>::type* __restrict__ tw4) {
@@ -790,17 +308,13 @@ k_fft_tile(const typename CT<R>::type* in, typename CT<R>::type* out, FftPass d,
     extern __shared__ __align__(16) unsigned char smem_raw[];
     __shared__ PreLds P;
     C* lds = reinterpret_cast<C*>(smem_raw);
-    // persistent one-row tiles are launched with 2^LGM / E threads (the host
-    // checks): a compile-time count lets the butterflies of one thread, which sit
-    // nt apart, share the twiddles their rows have in common
-    const int tid = threadIdx.x, nt = PF ? (1 << LGM) / E : (int)blockDim.x;
+    const int tid = threadIdx.x, nt = blockDim.x;
     constexpr int lgC = LGC;  // the tile's column count is part of the instance
     const int lgHb = d.lgHb;
     const int tile = 1 << (LGM + lgC + lgHb);
     // one-row complex64 tiles of 2^13-2^14 points: exchanges 0 and 1 in their own
     // layouts, the largest of which ends at tile + tile/8 (the host sizes LDS so)
     constexpr bool ONE = one_row_layouts<R, LGM, LGC>();
-    const int ldsEnd = ONE ? tile + (tile >> 3) : lds_ix(tile);
 
     if (d.usePre) {
         // constant indices: the argument is read in place (one entry per thread,
@@ -825,16 +339,6 @@ k_fft_tile(const typename CT<R>::type* in, typename CT<R>::type* out, FftPass d,
 
     const R scale = (R)d.outScale;
     const R scaleLo = (R)(d.outScale - (double)scale);
-    // One-row tiles keep every twiddle in LDS after the tile (split table, ~11 KiB):
-    // no global loads remain between a prefetch and its use.
-    const C* twl = tw;
-    if constexpr (PF) {
-        C* sTw = lds + ldsEnd;
-        for (int e = tid; e < SplitPlan<LGM>::total(); e += nt) sTw[e] = tw[e];
-        __syncthreads();
-        twl = sTw;
-    }
-
     auto tile_base = [&](uint64_t t, uint64_t& lo0, uint64_t& inBase, uint64_t& outBase) {
         const uint64_t loBlk = t & ((1ull << d.lgNLoBlk) - 1);
         const uint64_t r = t >> d.lgNLoBlk;
@@ -848,12 +352,12 @@ k_fft_tile(const typename CT<R>::type* in, typename CT<R>::type* out, FftPass d,
     auto prephase = [&](C* x, uint64_t t, int ti) {
         uint64_t lo0, inBase, outBase;
         tile_base(t, lo0, inBase, outBase);
-        stage0_pre<R0, E, LGM, LGC, !PF, PF ? TM_ROWS : TM_ANY>(x, d, inBase, P, pre, tw4, ti, nt, lds);
+        stage0_pre<R0, E, LGM, LGC, true, TM_ANY>(x, d, inBase, P, pre, tw4, ti, nt, lds);
     };
     // Transform the phased tile in registers (the last stage's outputs stay in x).
-    auto stages = [&](C* x, int ti, const C* twt) {
-        stage_compute<R0, E, LGM, LGC, 0, PF>(x, twt, ti, nt);
-        run_stages<LGM, LGC, 1, E, PF, ONE ? EX_ONE : EX_TILE>(x, lds, twt, ti, nt);
+    auto stages = [&](C* x, int ti) {
+        stage_compute<R0, E, LGM, LGC, 0>(x, tw, ti, nt);
+        run_stages<LGM, LGC, 1, E, ONE ? EX_ONE : EX_TILE>(x, lds, tw, ti, nt);
     };
     // Store the transformed tile t.
     // Staged store, first half: the last stage's outputs into LDS in natural order.
@@ -902,68 +406,24 @@ k_fft_tile(const typename CT<R>::type* in, typename CT<R>::type* out, FftPass d,
         store_lds(t, ti);
     };
 
-    if constexpr (!PF) {
-        // one tile per workgroup
-        const uint64_t t = blockIdx.x;
-        uint64_t lo0, inBase, outBase;
-        tile_base(t, lo0, inBase, outBase);
-        C x[E];
-        stage0_load<R0, E, LGM, LGC>(in, x, d, inBase, tid, nt);
-        if (d.conjLoad) {
+    // one tile per workgroup
+    const uint64_t t = blockIdx.x;
+    uint64_t lo0, inBase, outBase;
+    tile_base(t, lo0, inBase, outBase);
+    C x[E];
+    stage0_load<R0, E, LGM, LGC>(in, x, d, inBase, tid, nt);
+    if (d.conjLoad) {
 #pragma unroll
-            for (int i = 0; i < E; ++i) x[i].y = -x[i].y;
-        }
-        prephase(x, t, tid);
-        // an opaque copy of the thread id for the stages and the store: their
-        // index math would otherwise be computed early and held across the phases
-        // (8-element tiles; the 16-element one-row tile has no register left for it)
-        int t2 = tid;
-        if constexpr (E == 8) asm volatile("" : "+v"(t2));
-        stages(x, t2, twl);
-        store(x, t, t2);
-    } else {
-        // Persistent workgroups (tile t = blockIdx.x, + gridDim.x, ...): the next
-        // tile's inputs are loaded into registers before the current tile is
-        // transformed, so HBM reads overlap the LDS stages (the exchanges use
-        // LDS-only barriers, which leave those loads in flight).  Used for the
-        // one-row tiles that fill a CU's LDS alone.
-        uint64_t t = blockIdx.x;
-        C xn[E];
-        if (t < d.nTiles) {
-            uint64_t lo0, inBase, outBase;
-            tile_base(t, lo0, inBase, outBase);
-            stage0_load<R0, E, LGM, LGC>(in, xn, d, inBase, tid, nt);
-        }
-        while (t < d.nTiles) {
-            // Opaque per-iteration copies: index math derived from the thread id
-            // is the same for every tile; hoisted out of the loop it would pin
-            // dozens of registers across iterations.  The LDS twiddles are
-            // addressed from the shared array so that their loads stay LDS loads
-            // (a generic pointer would also count on the memory counter).
-            int ti = tid;
-            int twOff = ldsEnd;
-            asm volatile("" : "+v"(ti), "+v"(twOff));
-            const C* twt = lds + twOff;
-            C x[E];
-#pragma unroll
-            for (int i = 0; i < E; ++i) x[i] = xn[i];
-            // (no conjLoad here: it belongs to four-step halves, and the
-            // one-row tiles sit at 128 VGPRs already)
-            // the phase-table loads wait on the memory counter, which completes in
-            // order: issue the next tile's loads after them
-            prephase(x, t, ti);
-            const uint64_t tn = t + gridDim.x;
-            if (tn < d.nTiles) {
-                uint64_t lo0, inBase, outBase;
-                tile_base(tn, lo0, inBase, outBase);
-                stage0_load<R0, E, LGM, LGC>(in, xn, d, inBase, ti, nt);
-            }
-            stages(x, ti, twt);
-            store(x, t, ti);
-            lds_barrier();  // the next tile's first exchange overwrites LDS
-            t = tn;
-        }
+        for (int i = 0; i < E; ++i) x[i].y = -x[i].y;
     }
+    prephase(x, t, tid);
+    // an opaque copy of the thread id for the stages and the store: their
+    // index math would otherwise be computed early and held across the phases
+    // (8-element tiles; the 16-element one-row tile has no register left for it)
+    int t2 = tid;
+    if constexpr (E == 8) asm volatile("" : "+v"(t2));
+    stages(x, t2);
+    store(x, t, t2);
 }
 
 // Two half transforms of one register field in one in-place pass (FtDefer):
@@ -1036,8 +496,8 @@ k_fft_fused(typename CT<R>::type* data, FftPass d, FftPass dD, FastDiag pre, int
     }
     // pending half: the four-step twiddle (d carries no phases and no input conjugation)
     stage0_pre<R0, E, LGM, LGC, true, TM_NONE>(x, d, base, P, pre, tw4, tid, nt, lds);
-    stage_compute<R0, E, LGM, LGC, 0, false>(x, tw, tid, nt);
-    run_stages<LGM, LGC, 1, E, false>(x, lds, tw, tid, nt);
+    stage_compute<R0, E, LGM, LGC, 0>(x, tw, tid, nt);
+    run_stages<LGM, LGC, 1, E>(x, lds, tw, tid, nt);
     if (conjMid) {
 #pragma unroll
         for (int i = 0; i < E; ++i) x[i].y = -x[i].y;
@@ -1050,8 +510,8 @@ k_fft_fused(typename CT<R>::type* data, FftPass d, FftPass dD, FastDiag pre, int
     int t2 = tid;
     asm volatile("" : "+v"(t2));
     stage0_pre<R0, E, LGM, LGC, false, STG ? TM_STAGED : TM_ANY>(x, dD, natBase, P, pre, tw4, t2, nt, lds);
-    stage_compute<R0, E, LGM, LGC, 0, false>(x, tw, t2, nt);
-    run_stages<LGM, LGC, 1, E, false>(x, lds, tw, t2, nt);
+    stage_compute<R0, E, LGM, LGC, 0>(x, tw, t2, nt);
+    run_stages<LGM, LGC, 1, E>(x, lds, tw, t2, nt);
     out_finish<E>(x, d, d.conjOut, scale, scaleLo);
     last_store<RL, E, LGM, LGC>(data, x, d, base, scale, scaleLo, t2, nt);
 }
@@ -1078,6 +538,19 @@ __global__ void k_dft_naive(const typename CT<R>::type* in, typename CT<R>::type
         }
         out[g] = cmk<C>(ax * scale, ay * scale);  // accumulated in FP64, rounded once
     }
+}
+
+int device_cus() {
+    static std::map<int, int> cached;
+    int dev = 0;
+    HIPCHK(hipGetDevice(&dev));
+    std::lock_guard<std::mutex> lk(g_devCacheMu);
+    auto it = cached.find(dev);
+    if (it != cached.end()) return it->second;
+    int v = 0;
+    HIPCHK(hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev));
+    cached[dev] = v;
+    return v;
 }
 
 // ---------------------------------------------------------------- planning
@@ -1143,26 +616,6 @@ static bool fit_pass(const PassGeom& g, int prec, FftPass& d, bool allowBig, con
     return true;
 }
 
-// Workgroups of a kernel instance resident on the whole device at once.
-static uint64_t resident_blocks(const void* kfn, int threads, size_t lds) {
-    static std::map<std::tuple<int, const void*, int, size_t>, uint64_t> cache;
-    int dev = 0;
-    HIPCHK(hipGetDevice(&dev));
-    const auto key = std::make_tuple(dev, kfn, threads, lds);
-    {
-        std::lock_guard<std::mutex> lk(g_devCacheMu);
-        auto it = cache.find(key);
-        if (it != cache.end()) return it->second;
-    }
-    int cus = 0, per = 0;
-    HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kfn, threads, lds));
-    const uint64_t n = (uint64_t)std::max(per, 1) * (uint64_t)std::max(cus, 1);
-    std::lock_guard<std::mutex> lk(g_devCacheMu);
-    cache[key] = n;
-    return n;
-}
-
 // Kernel instances exist for the tile shapes fit_pass can produce: C = 2^LGC
 // columns (up to 256 bytes per row) with C*M within 64 KiB of LDS, or one whole
 // contiguous row (C = 1) of up to 2^14 complex64 / 2^13 complex128 points.
@@ -1192,6 +645,16 @@ static bool table_by_row(const FastDiag& pre, int fs, int fn) {
 
 static bool gen_affine_in_rows(const FastDiag& pre, int rowLo, int rowN);
 
+// What the row kernel takes: whole contiguous rows one after the other; tables read by row
+// and generic terms affine in the row coordinate.
+static bool row_shape(const FftPass& d) {
+    return d.lgHb == 0 && d.lgInR == 0 && d.lgOutR == 0 && d.lgNLoBlk == 0 && d.lgInH2 == d.lgM &&
+           d.lgOutH2 == d.lgM && d.nTiles == 1ull << d.lgNH2Blk;
+}
+static bool row_program(const FastDiag& pre, int lgm) {
+    return table_by_row(pre, 0, lgm) && (pre.ngen == 0 || gen_affine_in_rows(pre, 0, lgm));
+}
+
 template <typename R, int LGM, int LGC>
 static void launch_geom(CVDVContext* ctx, const typename CT<R>::type* in, typename CT<R>::type* out,
                         const FftPass& d, const FastDiag& pre, const typename CT<R>::type* tw,
@@ -1199,46 +662,45 @@ static void launch_geom(CVDVContext* ctx, const typename CT<R>::type* in, typena
     if constexpr (tile_instance<R, LGM, LGC>()) {
         FftPass dg = d;
         dg.genSteps = d.usePre && pre.ngen > 0 && gen_affine_in_rows(pre, d.lgInR, LGM) ? 1 : 0;
-        auto go = [&](auto kfn, int E, bool persistent) {
+        if constexpr (LGC == 0 && LGM >= FFT_ROW_LGM_MIN && LGM <= FFT_ROW_LGM_MAX && sizeof(R) == 4) {
+            // contiguous whole rows, in place: the row kernel (2^28: 0.80 ms without phases, 0.98
+            // by a tile of one workgroup a CU).  Rows elsewhere, and programs with a control or a
+            // one-bit term inside the row, stay with the tiles.
+            if (in == out && row_shape(d) && !d.tw4 && !d.conjLoad && d.conjIn == d.conjOut &&
+                (!d.usePre || row_program(pre, LGM))) {
+                RowArgs a{};
+                a.m = 1;
+                a.s[0].pre = d.usePre ? pre : FastDiag{};
+                a.s[0].inv = d.conjIn;
+                a.s[0].ctl = d.conjCtl;
+                a.useScale = d.useScale;
+                a.scale = d.outScale;
+                a.rows = d.nTiles;
+                fft_row_launch(ctx->stream, out, LGM, a, (const float2*)row_table(ctx, LGM));
+                return;
+            }
+        }
+        auto go = [&](auto kfn, int E) {
             if (tile / E > tile_threads_max<R, LGM, LGC>())
                 throw CvdvError{CVDV_ERR_UNSUPPORTED, "FFT tile larger than its kernel's workgroup bound"};
-            if (persistent && tile != (1 << LGM))
-                throw CvdvError{CVDV_ERR_UNSUPPORTED, "persistent FFT tile of more than one row"};
             if (lds > 64 * 1024)
                 HIPCHK(hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-            // persistent instances: as many workgroups as the device holds at once
-            const uint64_t grid =
-                persistent ? std::min<uint64_t>(blocks, resident_blocks((const void*)kfn, tile / E, lds)) : blocks;
-            hipLaunchKernelGGL(kfn, dim3((unsigned)grid), dim3(tile / E), lds, ctx->stream, in, out, dg, pre, tw,
-                               tw4);
+            hipLaunchKernelGGL(kfn, dim3((unsigned)blocks), dim3(tile / E), lds, ctx->stream, in, out, dg, pre, tw, tw4);
         };
-        // one-row complex64 tiles that fill a CU's LDS alone prefetch the next row
-        // and keep their (split) twiddles in LDS
-        // (the second pass of a four-step split, which carries the four-step
-        // twiddle, a pass that conjugates on load, and a program with a table not
-        // read by row run one tile per workgroup)
-        constexpr bool PF = LGC == 0 && LGM >= 13 && sizeof(R) == 4;
-        const bool pf = PF && !d.tw4 && !d.conjLoad && (!d.usePre || table_by_row(pre, d.lgInR, LGM));
         if constexpr (one_row_layouts<R, LGM, LGC>()) {
             if (tile != (1 << LGM))
                 throw CvdvError{CVDV_ERR_UNSUPPORTED, "one-row FFT tile of more than one row"};
             lds = (size_t)(tile + tile / 8) * sizeof(typename CT<R>::type);
         }
-        if (pf) {
-            tw = (const typename CT<R>::type*)split_table(ctx, LGM, sizeof(R) == 4 ? CVDV_MIXED : CVDV_C128);
-            lds += (size_t)SplitPlan<LGM>::total() * sizeof(typename CT<R>::type);
-        }
         if (lds > device_max_lds())
             throw CvdvError{CVDV_ERR_UNSUPPORTED, "FFT tile needs more LDS than the device has"};
         if constexpr (LGM == 14 && LGC == 0 && sizeof(R) == 4) {
             if (tile / 8 > 1024) {
-                if (pf) go(k_fft_tile<R, LGM, LGC, 16, PF>, 16, PF);
-                else go(k_fft_tile<R, LGM, LGC, 16, false>, 16, false);
+                go(k_fft_tile<R, LGM, LGC, 16>, 16);
                 return;
             }
         }
-        if (pf) go(k_fft_tile<R, LGM, LGC, 8, PF>, 8, PF);
-        else go(k_fft_tile<R, LGM, LGC, 8, false>, 8, false);
+        go(k_fft_tile<R, LGM, LGC, 8>, 8);
     } else {
         throw CvdvError{CVDV_ERR_UNSUPPORTED, "FFT tile shape without a kernel instance"};
     }
@@ -1715,15 +1177,66 @@ void fft_prepare(CVDVContext* ctx) {
         if (nb == 0 || nb > 28) continue;  // above 28 qubits the two-pass FFT refuses anyway
         for (int lg = 1; lg <= nb && lg <= 14; ++lg) (void)stage_table(ctx, lg, ctx->prec);
         if (ctx->prec == CVDV_MIXED)
-            for (int lg = 13; lg <= nb && lg <= 14; ++lg) (void)split_table(ctx, lg, ctx->prec);
+            for (int lg = FFT_ROW_LGM_MIN; lg <= nb && lg <= FFT_ROW_LGM_MAX; ++lg) (void)row_table(ctx, lg);
         (void)full_table(ctx, nb, ctx->prec);                   // four-step twiddles
         if (nb <= 12) (void)full_table(ctx, nb, CVDV_C128);     // direct DFT of tiny states
     }
 }
 
+// The chain of a contiguous row of 2^13 or 2^14 complex64 points.  Small states of 2^13
+// points stay with fft_chain.hip (no table builds); 2^14 points do not fit its tile
+// ([1,14], 12 gates: 380 us by single passes, 296 here).
+bool row_field(const CVDVContext* ctx, int sh, int nb) {
+    if (ctx->rec || ctx->prec != CVDV_MIXED || sh != 0 || nb < FFT_ROW_LGM_MIN || nb > FFT_ROW_LGM_MAX) return false;
+    return nb > 13 || ctx->totalQbt > FT_CHAIN_LG_SMALL;  // (2^13 points of a small state: fft_chain.hip)
+}
+
+// Every table is read by row and every generic term is affine in it; no pass of its own for
+// terms beyond a program's capacities (it would run ahead of the chain).
+bool row_accepts(int nb, const DiagProg& p) {
+    const uint64_t row = bit_field(0, nb);
+    for (int i = 0; i < p.n; ++i) {
+        const DiagTerm& t = p.t[i];
+        if (t.c1 == 0.0 && t.c2 == 0.0 && t.c3 == 0.0) continue;
+        if (t.ctrl >= 0 && t.ctrl < nb) return false;
+        if (t.kind == DT_ZBIT ? t.sh1 < nb : (t.sh1 < nb && (t.sh1 != 0 || t.nb1 != nb))) return false;
+        if (t.kind == DT_BILIN && t.sh2 < nb) return false;  // (its fields are in order of their shifts)
+    }
+    return diag_fits(diag_fold_linear(p, 0, nb), row);
+}
+
+void fft_row_chain(CVDVContext* ctx, int nb, const FtChainStep* st, int m) {
+    const uint64_t row = bit_field(0, nb);
+    int maxNb = 0;
+    for (int r = 0; r < ctx->numReg; ++r) maxNb = std::max(maxNb, ctx->nq[r]);
+    // the programs' tables side by side; reserved first, since a grown arena starts empty
+    arena_reserve(ctx, (size_t)m * diag_arena_bound(maxNb, ctx->elemBytes()));
+    RowArgs a{};
+    a.m = m;
+    a.scale = 1.0;
+    a.rows = ctx->totalSize >> nb;
+    uint32_t off = 0;
+    for (int i = 0; i < m; ++i) {
+        bool act = false, folded = false;
+        const FastDiag pre =
+            compile_diag(ctx, diag_fold_linear(st[i].prog, 0, nb), act, st[i].scale, &folded, row, off, &off);
+        if (act && !row_program(pre, nb)) throw CvdvError{CVDV_ERR_STATE, "row chain with a program not read by row"};
+        if (act) a.s[i].pre = pre;
+        a.s[i].pre.arena = ctx->arena;
+        a.s[i].inv = st[i].inverse;
+        a.s[i].ctl = st[i].ctrl + 1;
+        if (!folded) a.scale *= st[i].scale;
+    }
+    a.useScale = a.scale != 1.0;
+    const int pid = prof_begin(ctx, KK_FFT_ROW);
+    fft_row_launch(ctx->stream, (float2*)ctx->state(), nb, a, (const float2*)row_table(ctx, nb));
+    HIPCHK(hipGetLastError());
+    prof_end(ctx, pid);
+}
+
 bool fft_turns(const CVDVContext* ctx, int sh, int nb, int ctrl) {
     if (ctx->rec || (ctrl >= sh && ctrl < sh + nb)) return false;
-    if (ctx->totalQbt <= FT_CHAIN_LG_SMALL) return chain_field(ctx, sh, nb);
+    if (ctx->totalQbt <= FT_CHAIN_LG_SMALL && !row_field(ctx, sh, nb)) return chain_field(ctx, sh, nb);
     const uint64_t N = 1ull << nb, S = 1ull << sh, total = ctx->totalSize;
     const PassGeom g1{(int)N, S, total / (N * S), 1, 0, N * S, S, 0, N * S, S};
     FftPass d{};

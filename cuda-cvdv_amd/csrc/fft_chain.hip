@@ -216,8 +216,8 @@ k_fft_chain(ChainArgs a, typename CT<R>::type* data, const typename CT<R>::type*
 #pragma unroll
             for (int j = 0; j < 8; ++j) x[j].y = -x[j].y;
         }
-        stage_compute<8, 8, LGM, LGC, 0, false>(x, tw, ti, ST);
-        run_stages<LGM, LGC, 1, 8, false, EX>(x, lds, tw, ti, ST);
+        stage_compute<8, 8, LGM, LGC, 0>(x, tw, ti, ST);
+        run_stages<LGM, LGC, 1, 8, EX>(x, lds, tw, ti, ST);
         to_rows<LGM, 8>(x);
         if (inv) {
 #pragma unroll
@@ -308,9 +308,16 @@ void chain_flush(CVDVContext* ctx) {
     if (ch.n == 0) return;
     const int sh = ch.sh, nb = ch.nb, m = ch.n;
     ch.n = 0;  // launched or, on an error, dropped
-    if (m == 1 && ctx->totalQbt > FT_CHAIN_LG_SMALL) {
+    const bool rows = row_field(ctx, sh, nb);
+    if (m == 1 && (rows || ctx->totalQbt > FT_CHAIN_LG_SMALL)) {
         const FtChainStep c = ch.st[0];
         fft_whole(ctx, sh, nb, c.inverse != 0, c.prog, c.scale, c.ctrl);
+        return;
+    }
+    if (rows) {
+        FtChainStep st[FT_CHAIN_MAX];  // (compiling may flush)
+        std::copy(ch.st, ch.st + m, st);
+        fft_row_chain(ctx, nb, st, m);
         return;
     }
     int lgC, lgHb;
@@ -359,17 +366,18 @@ void chain_flush(CVDVContext* ctx) {
 
 bool chain_field(const CVDVContext* ctx, int sh, int nb) {
     int lgC, lgHb;
-    return chain_tile(ctx, sh, nb, lgC, lgHb);
+    return row_field(ctx, sh, nb) || chain_tile(ctx, sh, nb, lgC, lgHb);
 }
 
 bool chain_accept(CVDVContext* ctx, int sh, int nb, bool inverse, const DiagProg& pre, double outScale,
                   int ctrl) {
     FtChain& ch = ctx->chain;
     const bool one = !ch.open || !ctx->fuseFt;
-    if ((one && ctx->totalQbt > FT_CHAIN_LG_SMALL) || !chain_field(ctx, sh, nb)) return false;
+    const bool rows = row_field(ctx, sh, nb);
+    if ((one && (rows || ctx->totalQbt > FT_CHAIN_LG_SMALL)) || !chain_field(ctx, sh, nb)) return false;
     int n = 0;
     for (int k = 0; k < pre.n; ++k) n += !term_idle(pre.t[k]);
-    if (n > FT_CHAIN_TERMS) return false;
+    if (rows ? !row_accepts(nb, pre) : n > FT_CHAIN_TERMS) return false;
     if (ch.n > 0 && (ch.sh != sh || ch.nb != nb || ch.n == FT_CHAIN_MAX)) chain_flush(ctx);
     ch.sh = sh;
     ch.nb = nb;

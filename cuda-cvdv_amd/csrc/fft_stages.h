@@ -57,21 +57,6 @@ template <int LGM> struct Plan {
     }
 };
 
-// Offsets of the split twiddle table (split_values) for stage s of a length-2^LGM
-// transform: the direct segment (L <= 64) or the a and b segments.
-template <int LGM> struct SplitPlan {
-    static constexpr int seg(int s) {  // entries of stage s
-        const int R = 1 << Plan<LGM>::lgr(s), L = 1 << (3 * s);
-        return s == 0 ? 0 : (L <= 64 ? L * (R - 1) : (L / 64) * (R - 1) + 64 * (R - 1));
-    }
-    static constexpr int off(int s) {
-        int o = 0;
-        for (int i = 0; i < s; ++i) o += seg(i);
-        return o;
-    }
-    static constexpr int total() { return off(Plan<LGM>::NST); }
-};
-
 // Stockham stage geometry.  A butterfly of a stage of radix RP (sub-length L = 2^lgL
 // already transformed) takes rows q + i*M/RP of column c in block hb and writes rows
 // ob + m*L, ob = hb*M + (q/L)*RP*L + (q mod L); every thread owns E/RP butterflies.
@@ -121,9 +106,7 @@ __device__ __forceinline__ void to_rows(C* x) {
 }
 
 // Twiddle the inputs of the butterflies in x (stage S, radix RP) and transform.
-// TWL: the twiddles are the split table staged in LDS (one-row tiles), else the
-// stage table in global memory.
-template <int RP, int E, int LGM, int LGC, int S, bool TWL, typename C>
+template <int RP, int E, int LGM, int LGC, int S, typename C>
 __device__ __forceinline__ void stage_compute(C* x, const C* __restrict__ tw, int tid, int nt) {
     constexpr int lgC = LGC;
     constexpr int NB = E / RP;
@@ -133,24 +116,9 @@ __device__ __forceinline__ void stage_compute(C* x, const C* __restrict__ tw, in
         if (lgL > 0) {
             const BflyPos p = bfly_pos<RP, LGM, E>(tid, k, nt, lgC);
             const int pq = p.q & ((1 << lgL) - 1);
-            if constexpr (!TWL) {
-                const C* t = tw + Plan<LGM>::off(S) + pq * (RP - 1);
+            const C* t = tw + Plan<LGM>::off(S) + pq * (RP - 1);
 #pragma unroll
-                for (int i = 1; i < RP; ++i) x[k * RP + i] = cmul(x[k * RP + i], t[i - 1]);
-            } else if constexpr (lgL <= 6) {
-                const C* t = tw + SplitPlan<LGM>::off(S) + pq;
-#pragma unroll
-                for (int i = 1; i < RP; ++i) x[k * RP + i] = cmul(x[k * RP + i], t[(i - 1) << lgL]);
-            } else {
-                constexpr int LA = (1 << lgL) / 64;
-                constexpr int OA = SplitPlan<LGM>::off(S);
-                constexpr int OB = OA + LA * (RP - 1);
-                const C* ta = tw + OA + (pq >> 6);
-                const C* tb = tw + OB + (pq & 63);
-#pragma unroll
-                for (int i = 1; i < RP; ++i)
-                    x[k * RP + i] = cmul(x[k * RP + i], cmul(ta[(i - 1) * LA], tb[(i - 1) * 64]));
-            }
+            for (int i = 1; i < RP; ++i) x[k * RP + i] = cmul(x[k * RP + i], t[i - 1]);
         }
         dft_r<RP, false>(x + k * RP);
     }
@@ -223,7 +191,7 @@ __device__ __forceinline__ void stage_read(const C* lds, C* x, int tid, int nt) 
 // Stages 1 .. NST-1: exchange the previous stage's outputs through LDS, then
 // twiddle and transform.
 // HELD: the last stage takes its twiddles from the registers w.
-template <int LGM, int LGC, int S, int E, bool TWL, int EX = EX_TILE, bool HELD = false, typename C>
+template <int LGM, int LGC, int S, int E, int EX = EX_TILE, bool HELD = false, typename C>
 __device__ __forceinline__ void run_stages(C* x, C* lds, const C* __restrict__ tw, int tid, int nt,
                                            const C* w = nullptr) {
     if constexpr (S < Plan<LGM>::NST) {
@@ -234,7 +202,7 @@ __device__ __forceinline__ void run_stages(C* x, C* lds, const C* __restrict__ t
         stage_read<RP, E, LGM, LGC, S - 1, EX>(lds, x, tid, nt);
         lds_barrier();
         if constexpr (HELD && S == Plan<LGM>::NST - 1) stage_compute_held<RP, E>(x, w);
-        else stage_compute<RP, E, LGM, LGC, S, TWL>(x, tw, tid, nt);
-        run_stages<LGM, LGC, S + 1, E, TWL, EX, HELD>(x, lds, tw, tid, nt, w);
+        else stage_compute<RP, E, LGM, LGC, S>(x, tw, tid, nt);
+        run_stages<LGM, LGC, S + 1, E, EX, HELD>(x, lds, tw, tid, nt, w);
     }
 }

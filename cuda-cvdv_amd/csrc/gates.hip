@@ -76,7 +76,7 @@ struct TabMake {
 
 struct TabMakeArgs {
     int n;
-    uint32_t total;
+    uint32_t first, total;  // entries of the arena
     TabMake t[CVDV_FAST_TABS];
     TabMember m[CVDV_MAX_TERMS];
 };
@@ -85,7 +85,7 @@ struct TabMakeArgs {
 // reduced and summed, then FP64 sin/cos, rounded once to the state's precision.
 template <typename C>
 __global__ void k_make_tables(C* __restrict__ arena, TabMakeArgs a) {
-    for (uint32_t e = blockIdx.x * blockDim.x + threadIdx.x; e < a.total; e += gridDim.x * blockDim.x) {
+    for (uint32_t e = a.first + blockIdx.x * blockDim.x + threadIdx.x; e < a.total; e += gridDim.x * blockDim.x) {
         int i = 0;
         while (i + 1 < a.n && e >= a.t[i + 1].off) ++i;
         const TabMake& t = a.t[i];
@@ -370,7 +370,7 @@ size_t diag_arena_bound(int maxNb, size_t elemBytes) {
 }
 
 FastDiag compile_diag(CVDVContext* ctx, const DiagProg& p, bool& active, double scale, bool* scaleFolded,
-                      uint64_t tileBits) {
+                      uint64_t tileBits, uint32_t first, uint32_t* end) {
     FastDiag f{};
     if (scaleFolded) *scaleFolded = false;
     active = false;
@@ -388,7 +388,7 @@ FastDiag compile_diag(CVDVContext* ctx, const DiagProg& p, bool& active, double 
         if (!term_is_identity(p.t[i]) && !term_tabulated(p.t[i])) f.gen[f.ngen++] = p.t[i];
 
     TabMakeArgs a{};
-    uint32_t off = 0;
+    uint32_t off = first;
     int nm = 0;
     for (int k = 0; k < ng; ++k) {
         const TabGroup& G = grp[k];
@@ -467,10 +467,12 @@ FastDiag compile_diag(CVDVContext* ctx, const DiagProg& p, bool& active, double 
         if (scaleFolded) *scaleFolded = true;
     }
     active = f.ntab > 0 || f.ngen > 0;
+    if (end) *end = off;
     if (a.n) {
+        a.first = first;
         a.total = off;
         arena_reserve(ctx, (size_t)off * ctx->elemBytes());
-        const unsigned blocks = (unsigned)((off + 255) / 256);
+        const unsigned blocks = (unsigned)((off - first + 255) / 256);
         if (ctx->prec == CVDV_C128)
             hipLaunchKernelGGL(k_make_tables<double2>, dim3(blocks), dim3(256), 0, ctx->stream,
                                (double2*)ctx->arena, a);

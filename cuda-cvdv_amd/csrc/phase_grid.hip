@@ -182,8 +182,8 @@ k_grid_rows(double2* __restrict__ A, const double2* __restrict__ spec, uint64_t 
             const double2 v = cmul(x[i], cmul(u0, step[(p0.hb << 3) + i]));
             x[i] = make_double2(v.x * (1.0 / N), -v.y * (1.0 / N));
         }
-        stage_compute<8, 8, LGM, 0, 0, false>(x, tw, ti, NT);
-        run_stages<LGM, 0, 1, 8, false, EX_ROWS>(x, lds, tw, ti, NT);
+        stage_compute<8, 8, LGM, 0, 0>(x, tw, ti, NT);
+        run_stages<LGM, 0, 1, 8, EX_ROWS>(x, lds, tw, ti, NT);
         stage_write<RL, 8, LGM, 0, NST - 1, EX_ROWS>(lds, x, ti, NT);
         lds_barrier();
 #pragma unroll

@@ -320,8 +320,8 @@ k_wigner_rows(void* __restrict__ outv, const C* __restrict__ X, uint64_t S, int 
     double2 x[8];
     stage_read<R0, 8, LGM, 0, 0, EX_ROWS>(lds, x, tid, NT);
     lds_barrier();
-    stage_compute<R0, 8, LGM, 0, 0, false>(x, tw, tid, NT);
-    run_stages<LGM, 0, 1, 8, false, EX_ROWS>(x, lds, tw, tid, NT);
+    stage_compute<R0, 8, LGM, 0, 0>(x, tw, tid, NT);
+    run_stages<LGM, 0, 1, 8, EX_ROWS>(x, lds, tw, tid, NT);
     const double w = dx / PI;
 #pragma unroll
     for (int k = 0; k < 8 / RL; ++k) {
@@ -388,8 +388,8 @@ k_husimi_rows(double* __restrict__ acc, const C* __restrict__ X, uint64_t S, int
         }
 #pragma unroll
         for (int i = 0; i < 8; ++i) x[i] = make_double2(x[i].x * w[i], x[i].y * w[i]);
-        stage_compute<R0, 8, LGM, 0, 0, false>(x, tw, ti, NT);
-        run_stages<LGM, 0, 1, 8, false, EX_ROWS, true>(x, lds, tw, ti, NT, wl);
+        stage_compute<R0, 8, LGM, 0, 0>(x, tw, ti, NT);
+        run_stages<LGM, 0, 1, 8, EX_ROWS, true>(x, lds, tw, ti, NT, wl);
 #pragma unroll
         for (int i = 0; i < 8; ++i) sum[i] += x[i].x * x[i].x + x[i].y * x[i].y;
     }
