@@ -239,7 +239,7 @@ def run_c4(prec, circuits, n_seq, steps):
 # Sources each counter summary's kernels are compiled from (the phase programs
 # they apply come from gates.hip).  A summary records their fingerprint; a figure
 # is read from it only while the sources still match.
-FFT_SOURCES = ["fft.hip", "fft_bfly.h", "fft_stages.h", "fft_pass.h", "fft_row.hip", "fft_row.h", "diag_fast.h", "cvdv_internal.h", "gates.hip"]
+FFT_SOURCES = ["fft.hip", "fft_bfly.h", "fft_stages.h", "fft_pass.h", "fft_row.hip", "fft_row.h", "fft_fused.hip", "fft_fused.h", "fft_radix16.h", "diag_fast.h", "cvdv_internal.h", "gates.hip"]
 BATCH_SOURCES = ["batch.hip", "fft_bfly.h", "diag_fast.h", "cvdv_internal.h", "gates.hip"]
 
 

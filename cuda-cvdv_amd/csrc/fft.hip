@@ -28,6 +28,7 @@
 
 #include "cvdv_internal.h"
 #include "fft_pass.h"
+#include "fft_fused.h"
 #include "fft_row.h"
 
 static const long double PI_L = 3.141592653589793238462643383279502884L;
@@ -263,25 +264,6 @@ size_t device_max_lds() {
     return (size_t)v;
 }
 
-// Last-stage outputs straight to global memory (rows q + m*M/RP of column c).
-template <int RP, int E, int LGM, int LGC, typename R, typename C>
-__device__ __forceinline__ void last_store(C* __restrict__ out, const C* v, const FftPass& d, uint64_t outBase,
-                                           R scale, R scaleLo, int tid, int nt) {
-    constexpr int NB = E / RP;
-    constexpr int LGR = RP == 8 ? 3 : (RP == 4 ? 2 : 1);
-    constexpr int lgMq = LGM - LGR;
-#pragma unroll
-    for (int k = 0; k < NB; ++k) {
-        const BflyPos p = bfly_pos<RP, LGM, E>(tid, k, nt, LGC);
-        const uint64_t g0 = outBase + ((uint64_t)p.hb << d.lgOutH2) + p.c;
-#pragma unroll
-        for (int m = 0; m < RP; ++m) {
-            const int row = p.q + (m << lgMq);
-            out[g0 + ((uint64_t)row << d.lgOutR)] = v[k * RP + m];
-        }
-    }
-}
-
 // One-row complex64 tiles of 2^13-2^14 points lay out their first two exchanges
 // apart from the others (ex_lay); their LDS ends at tile + tile/8.
 template <typename R, int LGM, int LGC>
@@ -311,7 +293,6 @@ k_fft_tile(const typename CT<R>::type* in, typename CT<R>::type* out, FftPass d,
     const int tid = threadIdx.x, nt = blockDim.x;
     constexpr int lgC = LGC;  // the tile's column count is part of the instance
     const int lgHb = d.lgHb;
-    const int tile = 1 << (LGM + lgC + lgHb);
     // one-row complex64 tiles of 2^13-2^14 points: exchanges 0 and 1 in their own
     // layouts, the largest of which ends at tile + tile/8 (the host sizes LDS so)
     constexpr bool ONE = one_row_layouts<R, LGM, LGC>();
@@ -961,7 +942,9 @@ static void launch_fused_geom(CVDVContext* ctx, typename CT<R>::type* data, cons
         // workgroups per CU
         FftPass dDg = dD;
         dDg.genSteps = dD.usePre && pre.ngen > 0 && gen_affine_in_rows(pre, dD.lgInR, LGM) ? 1 : 0;
-        if constexpr (LGC > 0) {
+        // (complex64 digits of 2^7 points in whole runs: fft_fused.hip)
+        constexpr bool two = sizeof(R) == 4 && LGM == FUSE2_LGM && LGC == FUSE2_LGC;
+        if constexpr (LGC > 0 && !two) {
             const bool gen = sizeof(R) == 8 || pre.ngen == 0 || dDg.genSteps;
             if (!dD.usePre || (tile_tables_by_row(pre, dD) && gen)) {
                 hipLaunchKernelGGL((k_fft_fused<R, LGM, LGC, 8, true>), dim3((unsigned)blocks), dim3(tile / 8), lds,
@@ -1004,6 +987,19 @@ static void launch_fused(CVDVContext* ctx, const FftPass& d, const FftPass& dD, 
     const size_t lds = lds_bytes(tile, sizeof(C));
     C* data = (C*)ctx->state();
     const int pid = prof_begin(ctx, KK_FFT_FUSED);
+    if constexpr (sizeof(R) == 4) {
+        // two stages a digit where the instance's rules hold (fft_fused.hip)
+        if (d.lgM == FUSE2_LGM) {
+            FusedArgs a{dd, dD, conjMid, swapSh, swapLo, swapHi};
+            a.dD.genSteps = dD.usePre && pre.ngen > 0 && gen_affine_in_rows(pre, dD.lgInR, d.lgM) ? 1 : 0;
+            if ((!dD.usePre || (tile_tables_by_row(pre, dD) && (pre.ngen == 0 || a.dD.genSteps))) &&
+                fft_fused2_launch(ctx->stream, data, a, pre, (const C*)full_table(ctx, d.lgM, prec), tw4, (unsigned)blocks)) {
+                HIPCHK(hipGetLastError());
+                prof_end(ctx, pid);
+                return;
+            }
+        }
+    }
     switch (d.lgM) {
 #define CVDV_FUSE_M(L) \
     case L: launch_fused_lgm<R, L>(ctx, data, dd, dD, pre, conjMid, swapSh, swapLo, swapHi, tw, tw4, blocks, tile, lds); break;
@@ -1179,6 +1175,7 @@ void fft_prepare(CVDVContext* ctx) {
         if (ctx->prec == CVDV_MIXED)
             for (int lg = FFT_ROW_LGM_MIN; lg <= nb && lg <= FFT_ROW_LGM_MAX; ++lg) (void)row_table(ctx, lg);
         (void)full_table(ctx, nb, ctx->prec);                   // four-step twiddles
+        if (ctx->prec == CVDV_MIXED) (void)full_table(ctx, FUSE2_LGM, CVDV_MIXED);
         if (nb <= 12) (void)full_table(ctx, nb, CVDV_C128);     // direct DFT of tiny states
     }
 }

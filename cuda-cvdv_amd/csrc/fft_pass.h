@@ -469,3 +469,22 @@ __device__ __forceinline__ void out_finish(C* x, const FftPass& d, int conj, R s
         for (int i = 0; i < E; ++i) x[i].y = -x[i].y;
     }
 }
+
+// Last-stage outputs straight to global memory (rows q + m*M/RP of column c).
+template <int RP, int E, int LGM, int LGC, typename R, typename C>
+__device__ __forceinline__ void last_store(C* __restrict__ out, const C* v, const FftPass& d, uint64_t outBase,
+                                           R scale, R scaleLo, int tid, int nt) {
+    constexpr int NB = E / RP;
+    constexpr int LGR = RP == 8 ? 3 : (RP == 4 ? 2 : 1);
+    constexpr int lgMq = LGM - LGR;
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {
+        const BflyPos p = bfly_pos<RP, LGM, E>(tid, k, nt, LGC);
+        const uint64_t g0 = outBase + ((uint64_t)p.hb << d.lgOutH2) + p.c;
+#pragma unroll
+        for (int m = 0; m < RP; ++m) {
+            const int row = p.q + (m << lgMq);
+            out[g0 + ((uint64_t)row << d.lgOutR)] = v[k * RP + m];
+        }
+    }
+}
