@@ -355,7 +355,7 @@ void chain_flush(CVDVContext* ctx);                        // launch what was co
 // Contiguous complex64 rows of 2^13 and 2^14 points (fft_row.hip): fields whose transforms
 // the row kernel chains, the programs it takes, and one launch of a chain.
 bool row_field(const CVDVContext* ctx, int sh, int nb);
-bool row_accepts(int nb, const DiagProg& p);
+bool row_accepts(const CVDVContext* ctx, int nb, const DiagProg& p);
 void fft_row_chain(CVDVContext* ctx, int nb, const FtChainStep* st, int m);
 // fft.hip: a transform by itself (halves kept pending, or whole)
 void fft_whole(CVDVContext* ctx, int sh, int nb, bool inverse, const DiagProg& pre, double outScale, int ctrl = -1);

@@ -192,36 +192,37 @@ const void* fft_stage_table(TwiddleCache*& tcp, int logM, int prec) {
     return d;
 }
 
-// Twiddles of the row kernel (fft_row.hip): W_1024^{j p} of the middle stage (p < 32), then
-// W_M^{j t}, t < M/32, of the last as W_{M/32}^{j a} W_M^{j b}, t = 32 a + b; j-major.
-static void row_values(int lgm, std::vector<double>& re, std::vector<double>& im, std::vector<size_t>& segs) {
-    const uint64_t M = 1ull << lgm, RL = M >> 10;
+// Twiddles of the row kernel (fft_row.hip), E elements a thread: W_{E^2}^{j p} of the middle
+// stage (p < E), then W_M^{j t}, t < M/E, of the last as W_{M/E}^{j a} W_M^{j b}, t = E a + b;
+// j-major.
+static void row_values(int lgm, int lge, std::vector<double>& re, std::vector<double>& im, std::vector<size_t>& segs) {
+    const uint64_t M = 1ull << lgm, E = 1ull << lge, RL = M / (E * E);
     auto put = [&](uint64_t e, uint64_t N) {
         double c, s;
         host_twiddle(e, N, c, s);
         re.push_back(c);
         im.push_back(s);
     };
-    for (uint64_t j = 1; j < 32; ++j)
-        for (uint64_t p = 0; p < 32; ++p) put(j * p, 1024);
+    for (uint64_t j = 1; j < E; ++j)
+        for (uint64_t p = 0; p < E; ++p) put(j * p, E * E);
     segs.push_back(re.size());
     for (uint64_t j = 1; j < RL; ++j)
-        for (uint64_t a = 0; a < RL; ++a) put(j * a, M / 32);
+        for (uint64_t a = 0; a < RL; ++a) put(j * a, M / E);
     segs.push_back(re.size());
     for (uint64_t j = 1; j < RL; ++j)
-        for (uint64_t b = 0; b < 32; ++b) put(j * b, M);
+        for (uint64_t b = 0; b < E; ++b) put(j * b, M);
 }
 
-static const void* row_table(CVDVContext* ctx, int lgm) {
+static const void* row_table(CVDVContext* ctx, int lgm, int prec) {
     TwiddleCache* tc = cache(ctx);
-    const TwKey key{lgm + 1000, CVDV_MIXED};
+    const TwKey key{lgm + 1000, prec};
     auto it = tc->stage.find(key);
     if (it != tc->stage.end()) return it->second;
     if (ctx->capturing) throw CvdvError{CVDV_ERR_UNSUPPORTED, "FFT table not prepared before the graph capture"};
     std::vector<double> re, im;
     std::vector<size_t> segs;
-    row_values(lgm, re, im, segs);
-    void* d = upload_table(re, im, CVDV_MIXED, segs);
+    row_values(lgm, row_lge_of(prec == CVDV_C128), re, im, segs);
+    void* d = upload_table(re, im, prec, segs);
     tc->stage[key] = d;
     return d;
 }
@@ -643,10 +644,11 @@ static void launch_geom(CVDVContext* ctx, const typename CT<R>::type* in, typena
     if constexpr (tile_instance<R, LGM, LGC>()) {
         FftPass dg = d;
         dg.genSteps = d.usePre && pre.ngen > 0 && gen_affine_in_rows(pre, d.lgInR, LGM) ? 1 : 0;
-        if constexpr (LGC == 0 && LGM >= FFT_ROW_LGM_MIN && LGM <= FFT_ROW_LGM_MAX && sizeof(R) == 4) {
-            // contiguous whole rows, in place: the row kernel (2^28: 0.80 ms without phases, 0.98
-            // by a tile of one workgroup a CU).  Rows elsewhere, and programs with a control or a
-            // one-bit term inside the row, stay with the tiles.
+        constexpr bool c128 = sizeof(R) == 8;
+        if constexpr (LGC == 0 && row_instance(c128, LGM)) {
+            // contiguous whole rows, in place: the row kernel (2^28 complex64: 0.80 ms without
+            // phases, 0.98 by a tile of one workgroup a CU).  Rows elsewhere, and programs with a
+            // control or a one-bit term inside the row, stay with the tiles.
             if (in == out && row_shape(d) && !d.tw4 && !d.conjLoad && d.conjIn == d.conjOut &&
                 (!d.usePre || row_program(pre, LGM))) {
                 RowArgs a{};
@@ -657,7 +659,7 @@ static void launch_geom(CVDVContext* ctx, const typename CT<R>::type* in, typena
                 a.useScale = d.useScale;
                 a.scale = d.outScale;
                 a.rows = d.nTiles;
-                fft_row_launch(ctx->stream, out, LGM, a, (const float2*)row_table(ctx, LGM));
+                fft_row_launch(ctx->stream, out, c128, LGM, a, row_table(ctx, LGM, c128 ? CVDV_C128 : CVDV_MIXED));
                 return;
             }
         }
@@ -1172,25 +1174,30 @@ void fft_prepare(CVDVContext* ctx) {
         const int nb = ctx->nq[r];
         if (nb == 0 || nb > 28) continue;  // above 28 qubits the two-pass FFT refuses anyway
         for (int lg = 1; lg <= nb && lg <= 14; ++lg) (void)stage_table(ctx, lg, ctx->prec);
-        if (ctx->prec == CVDV_MIXED)
-            for (int lg = FFT_ROW_LGM_MIN; lg <= nb && lg <= FFT_ROW_LGM_MAX; ++lg) (void)row_table(ctx, lg);
+        for (int lg = 12; lg <= nb && lg <= 14; ++lg)
+            if (row_instance(ctx->prec == CVDV_C128, lg)) (void)row_table(ctx, lg, ctx->prec);
         (void)full_table(ctx, nb, ctx->prec);                   // four-step twiddles
         if (ctx->prec == CVDV_MIXED) (void)full_table(ctx, FUSE2_LGM, CVDV_MIXED);
         if (nb <= 12) (void)full_table(ctx, nb, CVDV_C128);     // direct DFT of tiny states
     }
 }
 
-// The chain of a contiguous row of 2^13 or 2^14 complex64 points.  Small states of 2^13
-// points stay with fft_chain.hip (no table builds); 2^14 points do not fit its tile
-// ([1,14], 12 gates: 380 us by single passes, 296 here).
+// The fields whose gates run as chains of rows.  Small states of 2^12 and 2^13 points stay with
+// fft_chain.hip (no table builds); 2^14 points do not fit its tile ([1,14], 12 gates: 380 us
+// by single passes, 296 here).
 bool row_field(const CVDVContext* ctx, int sh, int nb) {
-    if (ctx->rec || ctx->prec != CVDV_MIXED || sh != 0 || nb < FFT_ROW_LGM_MIN || nb > FFT_ROW_LGM_MAX) return false;
-    return nb > 13 || ctx->totalQbt > FT_CHAIN_LG_SMALL;  // (2^13 points of a small state: fft_chain.hip)
+    if (ctx->rec || sh != 0 || !row_instance(ctx->prec == CVDV_C128, nb)) return false;
+    return nb > 13 || ctx->totalQbt > FT_CHAIN_LG_SMALL;
+}
+
+// The program as a row's pass compiles it (fft_run's rule).
+static DiagProg row_prog(const CVDVContext* ctx, const DiagProg& p, int nb) {
+    return ctx->prec == CVDV_MIXED ? diag_fold_linear(p, 0, nb) : p;
 }
 
 // Every table is read by row and every generic term is affine in it; no pass of its own for
 // terms beyond a program's capacities (it would run ahead of the chain).
-bool row_accepts(int nb, const DiagProg& p) {
+bool row_accepts(const CVDVContext* ctx, int nb, const DiagProg& p) {
     const uint64_t row = bit_field(0, nb);
     for (int i = 0; i < p.n; ++i) {
         const DiagTerm& t = p.t[i];
@@ -1199,7 +1206,7 @@ bool row_accepts(int nb, const DiagProg& p) {
         if (t.kind == DT_ZBIT ? t.sh1 < nb : (t.sh1 < nb && (t.sh1 != 0 || t.nb1 != nb))) return false;
         if (t.kind == DT_BILIN && t.sh2 < nb) return false;  // (its fields are in order of their shifts)
     }
-    return diag_fits(diag_fold_linear(p, 0, nb), row);
+    return diag_fits(row_prog(ctx, p, nb), row);
 }
 
 void fft_row_chain(CVDVContext* ctx, int nb, const FtChainStep* st, int m) {
@@ -1216,7 +1223,7 @@ void fft_row_chain(CVDVContext* ctx, int nb, const FtChainStep* st, int m) {
     for (int i = 0; i < m; ++i) {
         bool act = false, folded = false;
         const FastDiag pre =
-            compile_diag(ctx, diag_fold_linear(st[i].prog, 0, nb), act, st[i].scale, &folded, row, off, &off);
+            compile_diag(ctx, row_prog(ctx, st[i].prog, nb), act, st[i].scale, &folded, row, off, &off);
         if (act && !row_program(pre, nb)) throw CvdvError{CVDV_ERR_STATE, "row chain with a program not read by row"};
         if (act) a.s[i].pre = pre;
         a.s[i].pre.arena = ctx->arena;
@@ -1226,7 +1233,7 @@ void fft_row_chain(CVDVContext* ctx, int nb, const FtChainStep* st, int m) {
     }
     a.useScale = a.scale != 1.0;
     const int pid = prof_begin(ctx, KK_FFT_ROW);
-    fft_row_launch(ctx->stream, (float2*)ctx->state(), nb, a, (const float2*)row_table(ctx, nb));
+    fft_row_launch(ctx->stream, ctx->state(), ctx->prec == CVDV_C128, nb, a, row_table(ctx, nb, ctx->prec));
     HIPCHK(hipGetLastError());
     prof_end(ctx, pid);
 }

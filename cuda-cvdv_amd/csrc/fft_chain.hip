@@ -236,9 +236,10 @@ k_fft_chain(ChainArgs a, typename CT<R>::type* data, const typename CT<R>::type*
 // every transform goes through here (gates alone, us, table path against chains: [1,10]
 // complex128 135 / 74, [8,8] 432 / 189, [1,10,10] 580 / 442, mixed 509 / 370).  Above,
 // HBM passes are the cost: only gates with several transforms of a field whose tile
-// keeps whole runs, and no more than 2^12 elements ([1,12,12] complex128 7.22 / 6.59 ms,
-// [14,12] mixed 9.89 / 8.92; runs of 64 bytes lose, [10,14] mixed 2.39 / 2.48, as do
-// tiles of 2^13, [14,13] mixed 20.1 / 20.8).
+// keeps whole runs, and no more than 2^12 elements ([1,12,12] complex128 7.22 / 6.59 ms by its
+// contiguous register, [14,12] mixed 9.89 / 8.92; runs of 64 bytes lose, [10,14] mixed 2.39 / 2.48, as do
+// tiles of 2^13, [14,13] mixed 20.1 / 20.8).  Contiguous rows of row_instance lengths go
+// through fft_row.hip there.
 static bool chain_tile(const CVDVContext* ctx, int sh, int nb, int& lgC, int& lgHb) {
     const int T = ctx->totalQbt, lgW = ctx->prec == CVDV_C128 ? 4 : 5;
     const bool small = T <= FT_CHAIN_LG_SMALL;
@@ -377,7 +378,7 @@ bool chain_accept(CVDVContext* ctx, int sh, int nb, bool inverse, const DiagProg
     if ((one && (rows || ctx->totalQbt > FT_CHAIN_LG_SMALL)) || !chain_field(ctx, sh, nb)) return false;
     int n = 0;
     for (int k = 0; k < pre.n; ++k) n += !term_idle(pre.t[k]);
-    if (rows ? !row_accepts(nb, pre) : n > FT_CHAIN_TERMS) return false;
+    if (rows ? !row_accepts(ctx, nb, pre) : n > FT_CHAIN_TERMS) return false;
     if (ch.n > 0 && (ch.sh != sh || ch.nb != nb || ch.n == FT_CHAIN_MAX)) chain_flush(ctx);
     ch.sh = sh;
     ch.nb = nb;

@@ -7,11 +7,12 @@
 // e^{-2 pi i E / 32} as float constants.  Nearest roundings of cos and sin leave |w|^2 - 1
 // of up to 6e-8, which an inner product of 21 fixed constants per stage would turn into a
 // drift of the norm; each pair below is within an ulp of the exact value, and the uses of
-// one stage sum to 3e-8 over 32 elements.
-template <int E> struct W32 {
+// one stage sum to 4e-8 over 32 elements.
+template <typename R, int E> struct W32;
+template <int E> struct W32<float, E> {
     static constexpr int q = (E >> 3) & 3, r = E & 7;
     static constexpr float c1 = (E & 31) == 1 ? 0.9807852506637573f : 0.9807853102684021f;
-    static constexpr float s1 = (E & 31) == 1 ? 0.19509032368659973f : 0.19509030878543854f;
+    static constexpr float s1 = 0.19509032368659973f;
     static constexpr float c2 = (E & 31) == 6 || (E & 31) == 14 ? 0.9238795042037964f : 0.9238795638084412f;
     static constexpr float s2 = 0.3826834261417389f;
     static constexpr float c3 = 0.8314695954322815f, s3 = 0.5555702447891235f;
@@ -19,26 +20,35 @@ template <int E> struct W32 {
     static constexpr float s = r == 1 ? s1 : r == 2 ? s2 : r == 3 ? s3 : r == 5 ? c3 : r == 6 ? c2 : c1;
 };
 
-template <int E>
-__device__ __forceinline__ float2 mul_w32(float2 a) {
-    using W = W32<E>;
-    float2 t = a;
+template <int E> struct W32<double, E> {
+    static constexpr int q = (E >> 3) & 3, r = E & 7;
+    static constexpr double c1 = 0.98078528040323044913, s1 = 0.19509032201612826785;
+    static constexpr double c2 = 0.92387953251128675613, s2 = 0.38268343236508977173;
+    static constexpr double c3 = 0.83146961230254523708, s3 = 0.55557023301960222474;
+    static constexpr double c = r == 1 ? c1 : r == 2 ? c2 : r == 3 ? c3 : r == 5 ? s3 : r == 6 ? s2 : s1;
+    static constexpr double s = r == 1 ? s1 : r == 2 ? s2 : r == 3 ? s3 : r == 5 ? c3 : r == 6 ? c2 : c1;
+};
+
+template <int E, typename C>
+__device__ __forceinline__ C mul_w32(C a) {
+    using W = W32<decltype(C{}.x), E>;
+    C t = a;
     if constexpr (W::r == 4) {
         t.x = mul_rsqrt2(a.x + a.y);
         t.y = mul_rsqrt2(a.y - a.x);
     } else if constexpr (W::r != 0) {
-        t.x = fmaf(a.x, W::c, a.y * W::s);
-        t.y = fmaf(a.y, W::c, -(a.x * W::s));
+        t.x = fma(a.x, W::c, a.y * W::s);
+        t.y = fma(a.y, W::c, -(a.x * W::s));
     }
-    float2 u;
+    C u;
     u.x = W::q == 0 ? t.x : W::q == 1 ? t.y : W::q == 2 ? -t.x : -t.y;
     u.y = W::q == 0 ? t.y : W::q == 1 ? -t.x : W::q == 2 ? -t.y : t.x;
     return u;
 }
 
 // Inputs x[0], x[ST], .. x[15 ST] in order, outputs in order.
-template <int ST>
-__device__ __forceinline__ void dft16(float2* x) {
+template <int ST, typename C>
+__device__ __forceinline__ void dft16(C* x) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) dft4<false>(x[j * ST], x[(j + 4) * ST], x[(j + 8) * ST], x[(j + 12) * ST]);
     // x[(j + 4 m) ST] is output m of group j
@@ -58,7 +68,7 @@ __device__ __forceinline__ void dft16(float2* x) {
     for (int m = 0; m < 4; ++m)
 #pragma unroll
         for (int n = m + 1; n < 4; ++n) {
-            const float2 t = x[(4 * m + n) * ST];
+            const C t = x[(4 * m + n) * ST];
             x[(4 * m + n) * ST] = x[(4 * n + m) * ST];
             x[(4 * n + m) * ST] = t;
         }
