@@ -325,6 +325,8 @@ void fft_register(CVDVContext* ctx, int pshift, int nbits, bool inverse, const D
 // The field's transforms may take their direction from an index bit: each tile's pass
 // holds one value of it, or each thread's chain does.
 bool fft_turns(const CVDVContext* ctx, int sh, int nb, int ctrl);
+// The most terms a program may have in such a transform: a chain's where only chains turn.
+int fft_turn_terms(const CVDVContext* ctx, int sh, int nb);
 // largest dynamic LDS a workgroup may request on the current device
 size_t device_max_lds();
 int device_cus();

@@ -1238,9 +1238,18 @@ void fft_row_chain(CVDVContext* ctx, int nb, const FtChainStep* st, int m) {
     prof_end(ctx, pid);
 }
 
+// States whose fields turn in chains alone (elsewhere a one-pass plan does).
+static bool turns_in_chains(const CVDVContext* ctx, int sh, int nb) {
+    return ctx->totalQbt <= FT_CHAIN_LG_SMALL && !row_field(ctx, sh, nb);
+}
+
+int fft_turn_terms(const CVDVContext* ctx, int sh, int nb) {
+    return turns_in_chains(ctx, sh, nb) ? FT_CHAIN_TERMS : CVDV_MAX_TERMS;
+}
+
 bool fft_turns(const CVDVContext* ctx, int sh, int nb, int ctrl) {
     if (ctx->rec || (ctrl >= sh && ctrl < sh + nb)) return false;
-    if (ctx->totalQbt <= FT_CHAIN_LG_SMALL && !row_field(ctx, sh, nb)) return chain_field(ctx, sh, nb);
+    if (turns_in_chains(ctx, sh, nb)) return chain_field(ctx, sh, nb);
     const uint64_t N = 1ull << nb, S = 1ull << sh, total = ctx->totalSize;
     const PassGeom g1{(int)N, S, total / (N * S), 1, 0, N * S, S, 0, N * S, S};
     FftPass d{};
@@ -1258,9 +1267,10 @@ void fft_register(CVDVContext* ctx, int pshift, int nbits, bool inverse, const D
 }
 
 void fft_whole(CVDVContext* ctx, int sh, int nb, bool inverse, const DiagProg& pre, double outScale, int ctrl) {
-    const bool done = ctx->prec == CVDV_C128 ? fft_deferred<double>(ctx, sh, nb, inverse, pre, outScale)
-                                             : fft_deferred<float>(ctx, sh, nb, inverse, pre, outScale);
-    if (done) return;  // (never with ctrl: a field with a one-pass plan keeps no half pending)
+    // (halves have one direction: a control goes on to fft_run, which refuses plans without it)
+    const bool done = ctrl < 0 && (ctx->prec == CVDV_C128 ? fft_deferred<double>(ctx, sh, nb, inverse, pre, outScale)
+                                                          : fft_deferred<float>(ctx, sh, nb, inverse, pre, outScale));
+    if (done) return;
     if (FtDefer* rec = ctx->defer.find(sh)) settle_one(ctx, *rec);
     bool swapped;
     if (ctx->prec == CVDV_C128)

@@ -718,8 +718,8 @@ static void ft_turned(CVDVContext* ctx, int reg, bool inverse, int ctrl) {
     if (!ctx->rec) fft_settle_for(ctx, pre, (((uint64_t)1 << nb) - 1ull) << ctx->pshift[reg]);
     bool found = false;
     for (int i = 0; i < pre.n; ++i) found |= same_slot(pre.t[i], tw);
-    // (a chain's programs are shorter, and one with a control has no other path there)
-    if (!found && pre.n >= (ctrl >= 0 ? FT_CHAIN_TERMS : CVDV_MAX_TERMS)) {
+    const int cap = ctrl >= 0 ? fft_turn_terms(ctx, ctx->pshift[reg], nb) : CVDV_MAX_TERMS;
+    if (pre.n + (found ? 0 : 1) > cap) {
         launch_diag(ctx, pre);
         pre = DiagProg{};
     }
