@@ -442,17 +442,22 @@ static Bufs extract_slices(CVDVContext* ctx, int r, double2* X) {
 }
 
 // The rows kernels read the slices of a contiguous field from the state itself, those
-// of any other field from the extracted copy X.
+// of any other field from the extracted copy X.  Wigner sums read every slice for every pair
+// of rows: from 16 complex64 slices on, widening them once (the copy) costs less than widening
+// them at every load ([4,8] 33 us by the copy, 42 directly; [4,12] 145 and 173; [3,8] 34 and 30).
 struct RowsIn {
     const void* p;
     bool wide;  // double2 (else float2)
     int refl;
 };
 
-static bool rows_direct(const CVDVContext* ctx, int r) { return ctx->pshift[r] == 0; }
+static bool rows_direct(const CVDVContext* ctx, int r, bool wigner) {
+    const bool widen = wigner && ctx->prec == CVDV_MIXED && (ctx->totalSize >> ctx->nq[r]) >= 16;
+    return ctx->pshift[r] == 0 && !widen;
+}
 
-static RowsIn rows_input(CVDVContext* ctx, int r, double2* X) {
-    if (rows_direct(ctx, r)) return RowsIn{ctx->state(), ctx->prec == CVDV_C128, ctx->refl[r]};
+static RowsIn rows_input(CVDVContext* ctx, int r, bool wigner, double2* X) {
+    if (rows_direct(ctx, r, wigner)) return RowsIn{ctx->state(), ctx->prec == CVDV_C128, ctx->refl[r]};
     extract_slices(ctx, r, X);
     return RowsIn{X, true, 0};
 }
@@ -461,18 +466,38 @@ static RowsIn rows_input(CVDVContext* ctx, int r, double2* X) {
 // slices for the grid's size the sum is the time, and the tiles win.  Measured (us, rows
 // against tiles, integrand, transform and finalisation): N = 2^8: 31 / 40 at 16 slices,
 // 168 / 71 at 256; 2^10: 62 / 72 at 64, 199 / 132 at 256; 2^12: 148 / 529 at 16,
-// 317 / 722 at 64, 1102 / 1511 at 256.  The line is N/16 slices (16 for small grids).
+// 317 / 722 at 64, 1102 / 1511 at 256.  The line is N/16 slices (16 for small grids).  At 2^5 and
+// 2^6 points, whose 2 and 4 workgroups of one wave each sum several rows in turn, it is 8, or 4
+// where the slices are extracted first: 33 / 29 and 35 / 32 at 16 slices, 28 / 32 at 8 (33 / 31
+// extracted); 2^4 24 / 28 at 16.
 static bool wigner_by_rows(const CVDVContext* ctx, int r) {
     const int n = ctx->nq[r];
-    const uint64_t N = 1ull << n;
-    return n >= ROWS_LGM_MIN && n <= ROWS_LGM_MAX && (ctx->totalSize >> n) <= (N > 256 ? N / 16 : 16);
+    const uint64_t N = 1ull << n, S = ctx->totalSize >> n;
+    if (n < ROWS_LGM_MIN || n > ROWS_LGM_MAX) return false;
+    if (n == 5 || n == 6) return S <= (rows_direct(ctx, r, true) ? 8 : 4);
+    return S <= (N > 256 ? N / 16 : 16);
+}
+
+// A Husimi row's workgroup transforms its slices one after the other: below 2^9 points there
+// are too few rows to fill the chip, and with many slices the windowed batches win.  Measured
+// (us, rows against batches, contiguous and extracted fields): 2^3: 47 / 61 at 64 slices, 106 /
+// 106 at 256; 2^6: 38 / 43 at 8, 44 / 47 and 49 / 45 at 16, 71 / 58 at 64, 1860 / 380 at 1024; 2^7:
+// 49 / 51 and 54 / 48 at 16, 89 / 72 at 64; 2^8: 92 / 92 and 102 / 92 at 64, 278 / 305 and 310 / 304 at
+// 256; 2^9: 301 / 897 at 256.
+static bool husimi_by_rows(const CVDVContext* ctx, int r) {
+    const int n = ctx->nq[r];
+    const uint64_t S = ctx->totalSize >> n;
+    if (n < ROWS_LGM_MIN || n > ROWS_LGM_MAX) return false;
+    if (n >= 9) return true;
+    if (rows_direct(ctx, r, false)) return n == 8 || S <= (n == 3 ? 64 : 16);
+    return S <= (n == 8 ? 32 : n <= 4 ? 16 : 8);
 }
 
 // Device scratch of wigner_device: X (A c128), and rho, G, tmp (N2 c128 each) where
 // the rows kernels don't serve the register.
 static size_t wigner_scratch(const CVDVContext* ctx, int r) {
     const uint64_t N2 = 1ull << (2 * ctx->nq[r]), A = ctx->totalSize;
-    if (wigner_by_rows(ctx, r)) return rows_direct(ctx, r) ? 0 : A * 16;
+    if (wigner_by_rows(ctx, r)) return rows_direct(ctx, r, true) ? 0 : A * 16;
     return A * 16 + 3 * N2 * 16;
 }
 
@@ -480,7 +505,7 @@ static size_t wigner_scratch(const CVDVContext* ctx, int r) {
 static void wigner_device(CVDVContext* ctx, int r, void* dev, bool asComplex, double2* X) {
     ctx_flush(ctx);
     if (wigner_by_rows(ctx, r)) {
-        const RowsIn in = rows_input(ctx, r, X);
+        const RowsIn in = rows_input(ctx, r, true, X);
         const uint64_t S = ctx->totalSize >> ctx->nq[r];
         const double2* tw = (const double2*)fft_stage_table(ctx->tw, ctx->nq[r], CVDV_C128);
         rows_dispatch(ctx->nq[r], [&](auto lg) {
@@ -548,14 +573,14 @@ static void get_husimi_overlap(CVDVContext* ctx, int r, double* out, bool outOnD
     ctx_flush(ctx);
     const int n = ctx->nq[r], N = 1 << n;
     const uint64_t N2 = (uint64_t)N * N, A = ctx->totalSize, S = A >> n;
-    if (n >= ROWS_LGM_MIN && n <= ROWS_LGM_MAX) {
+    if (husimi_by_rows(ctx, r)) {
         // scratch: X (A, when the field is not contiguous) | acc (N2 doubles) | Q (N2 doubles)
-        const size_t xb = rows_direct(ctx, r) ? 0 : A * 16;
+        const size_t xb = rows_direct(ctx, r, false) ? 0 : A * 16;
         char* base = (char*)ctx_scratch(ctx, xb + (outOnDevice ? 1 : 2) * N2 * 8);
         double* acc = (double*)(base + xb);
         double* Q = outOnDevice ? out : acc + N2;
         const int pid = prof_begin(ctx, KK_OTHER);
-        const RowsIn in = rows_input(ctx, r, (double2*)base);
+        const RowsIn in = rows_input(ctx, r, false, (double2*)base);
         const double2* tw = (const double2*)fft_stage_table(ctx->tw, n, CVDV_C128);
         rows_dispatch(n, [&](auto lg) {
             constexpr int L = decltype(lg)::value, HB = 1 << rows_lg_hb<L>();
