@@ -123,6 +123,7 @@ __global__ void k_grid_pairs(double2* __restrict__ A, const double2* __restrict_
         const int i = ix[x], a = i - d, b = i + d;
         double re = 0.0, im = 0.0;
         if (a >= 0 && b < N) {
+#pragma unroll 4
             for (uint64_t s = s0; s < s1; ++s) {
                 const double2 u = phi[(x * S + s) * N + a], v = phi[(x * S + s) * N + b];
                 re += u.x * v.x + u.y * v.y;  // u conj(v)
@@ -349,13 +350,27 @@ struct GridScratch {
     }
 };
 
+// Traced pictures sum the slices one after the other in every row's workgroup: with more than
+// a few slices that serial chain is the time, unless the rows alone fill the chip, and the
+// batched transforms of k_grid_shift and k_grid_pairs win.  Measured (us, rows against
+// batches): 32 points of N = 2^6: 77 / 73 at 16 slices, 163 / 90 at 64, 1840 / 435 at 1024;
+// of 2^10: 114 / 109 at 16, 256 / 141 at 64; 128 points of 2^10: 279 / 221 at 64; 256 of 2^10:
+// 286 / 327 at 64, 853 / 1003 at 256; 128 of 2^12: 655 / 770 at 64; 256 of 2^9: 225 / 215 at 64,
+// 2331 / 2532 at 1024; 16 of 2^3: 73 / 77 at 32, 99 / 87 at 64.
+static bool wigner_grid_by_rows(int n, uint64_t S, int nx, int perSlice) {
+    if (n < ROWS_LGM_MIN || n > ROWS_LGM_MAX) return false;
+    const uint64_t work = (uint64_t)nx << n;
+    return perSlice || S <= (n == 3 ? 32 : 16) || (nx >= 256 && work >= (1ull << 17)) ||
+           (nx >= 128 && work >= (1ull << 18));
+}
+
 static void get_wigner_grid(CVDVContext* ctx, int r, const double* xs, int nx, const double* ps, int np,
                             int perSlice, int native, double* out) {
     const int n = ctx->nq[r], N = 1 << n, nd = N > 1 ? N / 2 : 1, K = 2 * nd;
     const double dx = ctx->dx[r];
     const uint64_t A = ctx->totalSize, S = A >> n;
     const uint64_t outBlocks = perSlice ? S : 1;
-    const bool rows = n >= ROWS_LGM_MIN && n <= ROWS_LGM_MAX;
+    const bool rows = wigner_grid_by_rows(n, S, nx, perSlice);
     // x chunk: a power of two (the batched FFT over the chunk's S rows per point
     // needs a power-of-two row count); the last chunk is padded with t = 0 rows.
     // The row kernels have no intermediate but the operand A.
