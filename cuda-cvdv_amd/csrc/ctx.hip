@@ -363,6 +363,15 @@ __device__ __forceinline__ void put_out(void* out, uint64_t total, uint64_t o, d
     }
 }
 
+// out = the state as it lies: canonical layout, nothing pending.  One element a thread: 2^20
+// complex64 widened in 5.1 us, 8.9 through k_put with an empty program.
+template <typename C, int OUT>
+__global__ void k_widen(void* __restrict__ out, const C* __restrict__ in, uint64_t total) {
+    for (uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; g < total;
+         g += (uint64_t)gridDim.x * blockDim.x)
+        put_out<OUT, C>(out, total, g, make_double2((double)in[g].x, (double)in[g].y));
+}
+
 // out = the state with its pending phases applied, canonical layout (nothing to move).
 template <typename C, int OUT, bool IN>
 __global__ void k_put(void* __restrict__ out, const C* __restrict__ in, uint64_t total, FastDiag p, int usep) {
@@ -477,6 +486,16 @@ template <int OUT>
 static void put_state(CVDVContext* ctx, void* dst, const DiagProg& p) {
     const uint64_t n = ctx->totalSize;
     const bool move = !ctx->canonical();
+    if (!move && !prog_active(p)) {
+        if (ctx->prec == CVDV_C128)
+            hipLaunchKernelGGL((k_widen<double2, OUT>), dim3(grid_for(n)), dim3(256), 0, ctx->stream, dst,
+                               (const double2*)ctx->state(), n);
+        else
+            hipLaunchKernelGGL((k_widen<float2, OUT>), dim3(grid_for(n)), dim3(256), 0, ctx->stream, dst,
+                               (const float2*)ctx->state(), n);
+        HIPCHK(hipGetLastError());
+        return;
+    }
     const MoveArgs a = move ? move_args(ctx) : MoveArgs{};
     with_program(ctx, p, [&](auto in, const FastDiag& f, bool act, int per) {
         constexpr bool IN = decltype(in)::value;
@@ -524,6 +543,18 @@ static void read_state(CVDVContext* ctx, void* dst) {
     bool act;
     if (!inplace_diag(ctx, ctx->pending, f, act) && !diag_fits(ctx->pending, 0)) ctx_flush(ctx);
     put_state<OUT>(ctx, dst, ctx->pending);
+}
+
+// Memory of the current device that double2 elements may be stored to: another device's
+// buffer, or one aligned to its doubles only, takes the runtime's copy.
+static bool kernel_destination(const void* p) {
+    hipPointerAttribute_t a;
+    int dev = 0;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess || hipGetDevice(&dev) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return a.type == hipMemoryTypeDevice && a.device == dev && ((uintptr_t)p & (sizeof(double2) - 1)) == 0;
 }
 
 // ---------------------------------------------------------------- graph capture
@@ -833,8 +864,15 @@ void cvdvGetState(CVDVContext* ctx, double* realOut, double* imagOut) {
     const uint64_t n = ctx->totalSize;
     double* d = (double*)ctx_scratch(ctx, 2 * n * sizeof(double));
     read_state<OUT_SPLIT>(ctx, d);
-    copy_to_host(ctx->stream, realOut, d, n * sizeof(double));
-    copy_to_host(ctx->stream, imagOut, d + n, n * sizeof(double));
+    if (n * sizeof(double) < HOST_COPY_MIN) {
+        // both behind one wait: 2^11 amplitudes 42 us, 51 with one each
+        HIPCHK(hipMemcpyAsync(realOut, d, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+        HIPCHK(hipMemcpyAsync(imagOut, d + n, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+        HIPCHK(hipStreamSynchronize(ctx->stream));
+    } else {
+        copy_to_host(ctx->stream, realOut, d, n * sizeof(double));
+        copy_to_host(ctx->stream, imagOut, d + n, n * sizeof(double));
+    }
     CVDV_CATCH()
 }
 
@@ -941,7 +979,16 @@ void cvdvGetStateDevice(CVDVContext* ctx, void* d_dst) {
         return;
     }
     CVDV_TRY
-    read_state<OUT_C128>(ctx, d_dst);
+    fft_settle(ctx);
+    const bool plain = ctx->canonical() && !prog_active(ctx->pending);
+    if (ctx->prec == CVDV_C128 && (plain || !kernel_destination(d_dst))) {
+        // nothing to apply, or a destination that only a copy may reach
+        ctx_materialize(ctx);
+        HIPCHK(hipMemcpyAsync(d_dst, ctx->state(), ctx->totalSize * sizeof(double2), hipMemcpyDeviceToDevice,
+                              ctx->stream));
+    } else {
+        read_state<OUT_C128>(ctx, d_dst);
+    }
     HIPCHK(hipStreamSynchronize(ctx->stream));
     CVDV_CATCH()
 }

@@ -63,6 +63,8 @@ struct DiagProg {
     DiagTerm t[CVDV_MAX_TERMS];
 };
 
+inline bool prog_active(const DiagProg& p) { return p.n > 0 || p.grev != 0.0; }
+
 __host__ __device__ inline double cvdv_frac(double r) { return r - rint(r); }
 
 __device__ __forceinline__ double diag_field_m(uint64_t g, int sh, int nb) {

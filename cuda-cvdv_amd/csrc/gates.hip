@@ -207,8 +207,6 @@ static unsigned grid_for(uint64_t total, unsigned block = 256) {
     return (unsigned)(b ? b : 1);
 }
 
-static inline bool prog_active(const DiagProg& p) { return p.n > 0 || p.grev != 0.0; }
-
 // ---------------------------------------------------------------- pending program
 DiagProg ctx_take_pending(CVDVContext* ctx) {
     DiagProg p = ctx->pending;
