@@ -146,7 +146,11 @@ __global__ void k_qubit(C* __restrict__ s, uint64_t npairs, int bit, double2 m00
             if (pid >= npairs) continue;
             const uint64_t i0 = ((pid & ~lowmask) << 1) | (pid & lowmask);
             const uint64_t i1 = i0 | (1ull << bit);
-            const double2 ad = phased<IN>(p, usep, i0, a[k]), bd = phased<IN>(p, usep, i1, b[k]);
+            double2 ad = make_double2((double)a[k].x, (double)a[k].y), bd = make_double2((double)b[k].x, (double)b[k].y);
+            if (usep) {
+                ad = phased<IN>(p, 1, i0, a[k]);
+                bd = phased<IN>(p, 1, i1, b[k]);
+            }
             const double2 t00 = cmul(m00, ad), t01 = cmul(m01, bd), t10 = cmul(m10, ad), t11 = cmul(m11, bd);
             s[i0] = cmk<C>(t00.x + t01.x, t00.y + t01.y);
             s[i1] = cmk<C>(t10.x + t11.x, t10.y + t11.y);
