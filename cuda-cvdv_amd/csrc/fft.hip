@@ -227,6 +227,29 @@ static const void* row_table(CVDVContext* ctx, int lgm, int prec) {
     return d;
 }
 
+// Twiddles of the two-stage fused kernel (fft_fused.hip): for each j and q those of a thread's
+// two butterflies, side by side.
+static const void* fuse2_table(CVDVContext* ctx) {
+    TwiddleCache* tc = cache(ctx);
+    const TwKey key{FUSE2_LGM + 2000, CVDV_MIXED};
+    auto it = tc->stage.find(key);
+    if (it != tc->stage.end()) return it->second;
+    if (ctx->capturing) throw CvdvError{CVDV_ERR_UNSUPPORTED, "FFT table not prepared before the graph capture"};
+    const uint64_t M = 1ull << FUSE2_LGM, Q = M / 16;
+    std::vector<double> re, im;
+    for (uint64_t j = 1; j < 8; ++j)
+        for (uint64_t q = 0; q < Q; ++q)
+            for (uint64_t k = 0; k < 2; ++k) {
+                double c, s;
+                host_twiddle(j * (q + k * Q), M, c, s);
+                re.push_back(c);
+                im.push_back(s);
+            }
+    void* d = upload_table(re, im, CVDV_MIXED);
+    tc->stage[key] = d;
+    return d;
+}
+
 static void* stage_table(CVDVContext* ctx, int logM, int prec) {
     if (ctx->capturing && (!ctx->tw || !ctx->tw->stage.count({logM, prec})))
         throw CvdvError{CVDV_ERR_UNSUPPORTED, "FFT table not prepared before the graph capture"};
@@ -995,7 +1018,7 @@ static void launch_fused(CVDVContext* ctx, const FftPass& d, const FftPass& dD, 
             FusedArgs a{dd, dD, conjMid, swapSh, swapLo, swapHi};
             a.dD.genSteps = dD.usePre && pre.ngen > 0 && gen_affine_in_rows(pre, dD.lgInR, d.lgM) ? 1 : 0;
             if ((!dD.usePre || (tile_tables_by_row(pre, dD) && (pre.ngen == 0 || a.dD.genSteps))) &&
-                fft_fused2_launch(ctx->stream, data, a, pre, (const C*)full_table(ctx, d.lgM, prec), tw4, (unsigned)blocks)) {
+                fft_fused2_launch(ctx->stream, data, a, pre, (const float4*)fuse2_table(ctx), tw4, (unsigned)blocks)) {
                 HIPCHK(hipGetLastError());
                 prof_end(ctx, pid);
                 return;
@@ -1177,7 +1200,7 @@ void fft_prepare(CVDVContext* ctx) {
         for (int lg = 12; lg <= nb && lg <= 14; ++lg)
             if (row_instance(ctx->prec == CVDV_C128, lg)) (void)row_table(ctx, lg, ctx->prec);
         (void)full_table(ctx, nb, ctx->prec);                   // four-step twiddles
-        if (ctx->prec == CVDV_MIXED) (void)full_table(ctx, FUSE2_LGM, CVDV_MIXED);
+        if (ctx->prec == CVDV_MIXED) (void)fuse2_table(ctx);
         if (nb <= 12) (void)full_table(ctx, nb, CVDV_C128);     // direct DFT of tiny states
     }
 }

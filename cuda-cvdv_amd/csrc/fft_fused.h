@@ -13,6 +13,6 @@ struct FusedArgs {
     int conjMid, swapSh, swapLo, swapHi;
 };
 
-// `tw`: W_128^e, e < 128.  False: no instance for this shape.
-bool fft_fused2_launch(hipStream_t stream, float2* data, const FusedArgs& a, const FastDiag& pre, const float2* tw,
+// `tw`: W_128^{j q}, W_128^{j (q + 8)} at (j - 1) 8 + q, 1 <= j < 8, q < 8.  False: no instance for this shape.
+bool fft_fused2_launch(hipStream_t stream, float2* data, const FusedArgs& a, const FastDiag& pre, const float4* tw,
                        const float2* tw4, unsigned blocks);

@@ -4,8 +4,8 @@
 // The tile kernel (k_fft_fused in fft.hip) takes such a digit in three stages of 8 elements a
 // thread (8 x 8 x 2): six stages and four exchanges a pass, 102 VALU instructions an
 // element, which is what bounds it.  With 16 elements a thread a digit is two stages, 16 x 8,
-// and one exchange: [14,14] complex64 (a copy of this shape takes 0.82 ms) 1.09 -> 0.97
-// ms a pass of displacements, 1.00 -> 0.91 of squeezing, 0.99 -> 0.89 of beam splitters.
+// and one exchange: [14,14] complex64 (a copy of this shape takes 0.82 ms), ms a gate of the strided
+// register: displacement 2.01 -> 1.81, squeezing 4.04 -> 3.61, beam splitter 4.03 -> 3.50.
 // complex64 in runs of 256 bytes only: in complex128 the 16 elements take 242 VGPRs, two
 // waves a SIMD, and [13,12] displacements went from 0.22 to 0.26 ms.
 
@@ -18,7 +18,7 @@
 __device__ constexpr int fuse2_at(int e) { return 8 * (e & 1) + (e >> 1); }
 
 // The digit's transform over a tile, the thread's rows q + e M/16 before and after.
-__device__ __forceinline__ void digit_fft(float2* x, float2* lds, const float2* __restrict__ tw, int tid) {
+__device__ __forceinline__ void digit_fft(float2* x, float2* lds, const float4* __restrict__ tw, int tid) {
     using C = float2;
     constexpr int LGM = FUSE2_LGM, LGC = FUSE2_LGC, M = 1 << LGM, QN = M / 16, NB = 2;
     const int c = tid & ((1 << LGC) - 1), q = (tid >> LGC) & (QN - 1), hb = tid >> (LGC + LGM - 4);
@@ -39,19 +39,15 @@ __device__ __forceinline__ void digit_fft(float2* x, float2* lds, const float2* 
         for (int e = 0; e < 16; ++e) y[e] = rd[(e * QN) << LGC];
     }
     lds_barrier();
-    // butterfly k sits at q + k QN: W_M^{j (q + k QN)} = W_M^{j q} W_16^{j k}
-    C w[8];
+    // butterfly k sits at q + k QN: W_M^{j (q + k QN)}, one rounded product each, both butterflies'
+    // in one load (as W_M^{j q} W_16^{j k} the second takes two products, and eight transforms of
+    // [14,5] are 5.07e-7 off instead of 4.40e-7; 4.77e-7 by 8 x 8 x 2)
 #pragma unroll
-    for (int j = 1; j < 8; ++j) w[j] = tw[j * q];
-#pragma unroll
-    for (int j = 1; j < 8; ++j) y[NB * j] = cmul(y[NB * j], w[j]);
-    y[3] = mul_w32<2>(cmul(y[3], w[1]));
-    y[5] = mul_w32<4>(cmul(y[5], w[2]));
-    y[7] = mul_w32<6>(cmul(y[7], w[3]));
-    y[9] = mul_w32<8>(cmul(y[9], w[4]));
-    y[11] = mul_w32<10>(cmul(y[11], w[5]));
-    y[13] = mul_w32<12>(cmul(y[13], w[6]));
-    y[15] = mul_w32<14>(cmul(y[15], w[7]));
+    for (int j = 1; j < 8; ++j) {
+        const float4 w = tw[(j - 1) * QN + q];
+        y[NB * j] = cmul(y[NB * j], make_float2(w.x, w.y));
+        y[NB * j + 1] = cmul(y[NB * j + 1], make_float2(w.z, w.w));
+    }
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
         C z[8];
@@ -68,7 +64,7 @@ __device__ __forceinline__ void digit_fft(float2* x, float2* lds, const float2* 
 // As k_fft_fused (fft.hip) where every table is read by row and the generic terms are affine in
 // the rows.
 __global__ void __launch_bounds__(FUSE2_THREADS, 5)
-k_fft_fused2(float2* data, FusedArgs a, FastDiag pre, const float2* __restrict__ tw, const float2* __restrict__ tw4) {
+k_fft_fused2(float2* data, FusedArgs a, FastDiag pre, const float4* __restrict__ tw, const float2* __restrict__ tw4) {
     using C = float2;
     constexpr int LGM = FUSE2_LGM, LGC = FUSE2_LGC;
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -128,7 +124,7 @@ k_fft_fused2(float2* data, FusedArgs a, FastDiag pre, const float2* __restrict__
     last_store<8, 16, LGM, LGC>(data, x, d, base, scale, scaleLo, t2, nt);
 }
 
-bool fft_fused2_launch(hipStream_t stream, float2* data, const FusedArgs& a, const FastDiag& pre, const float2* tw,
+bool fft_fused2_launch(hipStream_t stream, float2* data, const FusedArgs& a, const FastDiag& pre, const float4* tw,
                        const float2* tw4, unsigned blocks) {
     const int tile = 1 << (FUSE2_LGM + FUSE2_LGC + a.d.lgHb);
     const size_t lds = (size_t)tile * sizeof(float2);
