@@ -886,12 +886,8 @@ void cvdvGraphBegin(CVDVContext* ctx) {
     ctx_materialize(ctx);
     (void)ctx->other();  // both buffers exist before the capture
     int maxNb = 0;
-    bool rows = false;  // a chain of rows keeps the tables of all its programs
-    for (int r = 0; r < ctx->numReg; ++r) {
-        maxNb = std::max(maxNb, ctx->nq[r]);
-        rows |= row_field(ctx, 0, ctx->nq[r]);
-    }
-    arena_reserve(ctx, diag_arena_bound(maxNb, ctx->elemBytes()) * (rows ? FT_CHAIN_MAX : 1));
+    for (int r = 0; r < ctx->numReg; ++r) maxNb = std::max(maxNb, ctx->nq[r]);
+    arena_reserve(ctx, diag_arena_bound(maxNb, ctx->elemBytes()));
     fft_prepare(ctx);
     HIPCHK(hipStreamSynchronize(ctx->stream));
     for (int r = 0; r < ctx->numReg; ++r) {

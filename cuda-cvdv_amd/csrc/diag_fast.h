@@ -160,6 +160,9 @@ DiagProg diag_fold_linear(const DiagProg& p, int sh, int nb);
 // FP64 pass and no table pass of its own (with a table slot to spare).
 bool diag_fits(const DiagProg& p, uint64_t tileBits);
 
+// Table entries that compile_diag needs for a program that fits, at most.
+uint32_t diag_entries(const DiagProg& p, uint64_t tileBits);
+
 // Largest table arena compile_diag can need for registers of at most maxNb qubits.
 size_t diag_arena_bound(int maxNb, size_t elemBytes);
 

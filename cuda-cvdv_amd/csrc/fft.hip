@@ -1236,8 +1236,18 @@ void fft_row_chain(CVDVContext* ctx, int nb, const FtChainStep* st, int m) {
     const uint64_t row = bit_field(0, nb);
     int maxNb = 0;
     for (int r = 0; r < ctx->numReg; ++r) maxNb = std::max(maxNb, ctx->nq[r]);
-    // the programs' tables side by side; reserved first, since a grown arena starts empty
-    arena_reserve(ctx, (size_t)m * diag_arena_bound(maxNb, ctx->elemBytes()));
+    // the programs' tables side by side; reserved first, since a grown arena starts empty.  Never
+    // more than one program may ask for by itself (a capture reserves no more): steps whose
+    // tables together exceed that run one by one
+    uint64_t entries = 0;
+    for (int i = 0; i < m; ++i) entries += diag_entries(row_prog(ctx, st[i].prog, nb), row);
+    const size_t need = entries * ctx->elemBytes();
+    if (need > diag_arena_bound(maxNb, ctx->elemBytes())) {
+        for (int i = 0; i < m; ++i)
+            fft_whole(ctx, 0, nb, st[i].inverse != 0, st[i].prog, st[i].scale, st[i].ctrl);
+        return;
+    }
+    arena_reserve(ctx, need);
     RowArgs a{};
     a.m = m;
     a.scale = 1.0;

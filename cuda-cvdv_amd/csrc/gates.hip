@@ -379,6 +379,17 @@ size_t diag_arena_bound(int maxNb, size_t elemBytes) {
     return ((size_t)CVDV_FAST_TABS * ((size_t)1 << std::max(plain, merged)) + 1) * elemBytes;
 }
 
+uint32_t diag_entries(const DiagProg& p, uint64_t tileBits) {
+    TabGroup grp[CVDV_FAST_TABS + 1];
+    const int ng = group_tables(p, grp, tileBits);
+    uint32_t sum = 1, promoted = 0;  // a one-entry table, or a lone conditional term's entries twice
+    for (int k = 0; k < ng; ++k) {
+        sum += 1u << (grp[k].nb + grp[k].nsel);
+        if (grp[k].nm == 1 && grp[k].ctrl >= 0) promoted = std::max(promoted, 1u << grp[k].nb);
+    }
+    return sum + promoted;
+}
+
 FastDiag compile_diag(CVDVContext* ctx, const DiagProg& p, bool& active, double scale, bool* scaleFolded,
                       uint64_t tileBits, uint32_t first, uint32_t* end) {
     FastDiag f{};
