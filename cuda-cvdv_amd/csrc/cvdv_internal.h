@@ -72,12 +72,20 @@ __device__ __forceinline__ double diag_field_m(uint64_t g, int sh, int nb) {
     return (double)((int64_t)(2 * j) + 1 - ((int64_t)1 << nb));
 }
 
+// c1 m + c2 m^2 + c3 m^3 modulo 1: the linear part and the rest each reduced before they are
+// rounded (m and m^2 are exact).  A transform's own linear term reaches a thousand revolutions
+// at the edge; in one sum with a quadratic it would cost that its last digits.
+__device__ __forceinline__ double poly_rev(double c1, double c2, double c3, double m) {
+    const double m2 = m * m, q = fma(c3, m, c2);
+    return fma(c1, m, -rint(c1 * m)) + fma(q, m2, -rint(q * m2));
+}
+
 // One term's phase of element g in revolutions (modulo 1, not reduced in general).
 __device__ __forceinline__ double diag_term_rev(const DiagTerm& t, uint64_t g) {
     double v;
     if (t.kind == DT_POLY || t.kind == DT_LINF) {
         const double m = diag_field_m(g, t.sh1, t.nb1);
-        v = fma(fma(t.c3, m, t.c2), m, t.c1) * m;
+        v = poly_rev(t.c1, t.c2, t.c3, m);
     } else if (t.kind == DT_BILIN) {
         const double m1 = diag_field_m(g, t.sh1, t.nb1);
         const double m2 = diag_field_m(g, t.sh2, t.nb2);

@@ -59,8 +59,10 @@ template <typename R, int LGM, int LGC> constexpr int chain_block_lds() {
 // last digits ([1,1,1,1,12] state transfer: 1.7e-14 off instead of 3e-15).
 struct RowCubic {
     double a, c1, c2, c3;
+    // (the quadratic and cubic part, a thousand revolutions at the edge, reduced before it is rounded)
     __device__ __forceinline__ double at(double m) const {
-        return cvdv_frac(a * m) + cvdv_frac(fma(fma(c3, m, c2), m, c1) * m);
+        const double m2 = m * m, q = fma(c3, m, c2);
+        return cvdv_frac(a * m) + fma(c1, m, fma(q, m2, -rint(q * m2)));
     }
     __device__ __forceinline__ void linear(double c, double n4) {  // n4 = 4N
         c = cvdv_frac(c);
@@ -87,7 +89,9 @@ __device__ __forceinline__ RowCubic row_cubic(const ChainStep& st, uint32_t g, i
             const bool first = __builtin_amdgcn_readfirstlane(t.sh1) == sh;
             const int osh = __builtin_amdgcn_readfirstlane(first ? t.sh2 : t.sh1);
             const int onb = __builtin_amdgcn_readfirstlane(first ? t.nb2 : t.nb1);
-            f.linear(sg * t.c1 * chain_coord(g, osh, onb), 4.0 * N);
+            const double c = chain_coord(g, osh, onb), p = t.c1 * c;
+            f.linear(sg * p, 4.0 * N);
+            f.c1 += sg * fma(t.c1, c, -p);
         } else {
             f.linear(sg * t.c1, 4.0 * N);
             f.c2 += sg * t.c2;

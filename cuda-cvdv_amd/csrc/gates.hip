@@ -81,14 +81,6 @@ struct TabMakeArgs {
     TabMember m[CVDV_MAX_TERMS];
 };
 
-// c1 m + c2 m^2 + c3 m^3 modulo 1: the linear part and the rest each reduced before they are
-// rounded (m and m^2 are exact).  A transform's own linear term reaches a thousand revolutions
-// at the edge; in one sum with a quadratic it would cost that its last digits.
-__device__ __forceinline__ double table_rev(double c1, double c2, double c3, double m) {
-    const double m2 = m * m, q = fma(c3, m, c2);
-    return fma(c1, m, -rint(c1 * m)) + fma(q, m2, -rint(q * m2));
-}
-
 // e^{2 pi i phase(entry)} for every table entry: each member's angle in FP64,
 // reduced and summed, then FP64 sin/cos, rounded once to the state's precision.
 template <typename C>
@@ -106,9 +98,9 @@ __global__ void k_make_tables(C* __restrict__ arena, TabMakeArgs a) {
             double mv;
             if (M.vsel >= 0) {
                 const double m = ((choice >> M.vsel) & 1u) ? 1.0 : -1.0;
-                mv = M.kind == DT_ZBIT ? M.c1 * m : table_rev(M.c1, M.c2, M.c3, m);
+                mv = M.kind == DT_ZBIT ? M.c1 * m : poly_rev(M.c1, M.c2, M.c3, m);
             } else {
-                mv = M.kind == DT_ZBIT ? M.c1 * mf : table_rev(M.c1, M.c2, M.c3, mf);
+                mv = M.kind == DT_ZBIT ? M.c1 * mf : poly_rev(M.c1, M.c2, M.c3, mf);
             }
             if (M.csel >= 0 && ((choice >> M.csel) & 1u)) mv = -mv;
             v += cvdv_frac(mv);
