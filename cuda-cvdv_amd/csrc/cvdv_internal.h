@@ -351,7 +351,8 @@ void fft_settle(CVDVContext* ctx, bool mayAllocate = true);
 bool fft_defers(const CVDVContext* ctx, int sh, int nb);
 // Tile geometry the planner picks for field [sh, sh+nb) of the context's state
 // under cfg, folded into one number (equal numbers: the same passes); 0 when
-// the FFT of that field takes no tile pass (direct DFT of a tiny state).
+// the FFT of that field takes no tile pass (direct DFT of a tiny state).  Fields whose
+// transforms run as chains have one plan, whatever cfg says.
 uint64_t fft_plan_signature(const CVDVContext* ctx, int sh, int nb, const FftCfg& cfg);
 // A context of src's shape and precision in the canonical layout, its state
 // zeroed, nothing pending (the FFT autotuner times candidates on it).

@@ -1177,9 +1177,16 @@ bool fft_defers(const CVDVContext* ctx, int sh, int nb) {
     return four_step_geom(ctx->prec, total, sh, nb, f, cfg) && fusable(ctx, f, nb, cfg);
 }
 
+// States whose fields turn in chains alone (elsewhere a one-pass plan does).
+static bool turns_in_chains(const CVDVContext* ctx, int sh, int nb) {
+    return ctx->totalQbt <= FT_CHAIN_LG_SMALL && !row_field(ctx, sh, nb);
+}
+
 uint64_t fft_plan_signature(const CVDVContext* ctx, int sh, int nb, const FftCfg& cfg) {
     const uint64_t N = 1ull << nb, S = 1ull << sh, total = ctx->totalSize;
     if (total % (N * S) != 0) return 0;
+    // transforms that run as chains take none of cfg's choices
+    if (turns_in_chains(ctx, sh, nb) && chain_field(ctx, sh, nb)) return 500000;
     auto sig = [](const FftPass& d) { return (uint64_t)(d.lgC * 64 + d.lgHb * 4 + d.lgM / 8 + 1); };
     PassGeom g1{(int)N, S, total / (N * S), 1, 0, N * S, S, 0, N * S, S};
     FftPass d{};
@@ -1269,11 +1276,6 @@ void fft_row_chain(CVDVContext* ctx, int nb, const FtChainStep* st, int m) {
     fft_row_launch(ctx->stream, ctx->state(), ctx->prec == CVDV_C128, nb, a, row_table(ctx, nb, ctx->prec));
     HIPCHK(hipGetLastError());
     prof_end(ctx, pid);
-}
-
-// States whose fields turn in chains alone (elsewhere a one-pass plan does).
-static bool turns_in_chains(const CVDVContext* ctx, int sh, int nb) {
-    return ctx->totalQbt <= FT_CHAIN_LG_SMALL && !row_field(ctx, sh, nb);
 }
 
 int fft_turn_terms(const CVDVContext* ctx, int sh, int nb) {
