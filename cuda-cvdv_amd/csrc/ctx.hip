@@ -400,7 +400,7 @@ __global__ void __launch_bounds__(256) k_move(void* __restrict__ out, const C* _
     constexpr int PER = (1 << MOVE_TILE_BITS) / 256;
     const int tid = threadIdx.x, n = 1 << a.nb;
     uint64_t g0 = 0, mask = a.rest;
-    for (uint32_t b = blockIdx.x; mask && b; b >>= 1) {
+    for (uint32_t b = blockIdx.x + blockIdx.y * gridDim.x; mask && b; b >>= 1) {
         const uint64_t low = mask & (~mask + 1ull);
         if (b & 1u) g0 |= low;
         mask &= mask - 1ull;
@@ -502,9 +502,12 @@ static void put_state(CVDVContext* ctx, void* dst, const DiagProg& p) {
         const int usep = act ? 1 : 0;
         auto go = [&](auto* src) {
             using C = std::remove_const_t<std::remove_pointer_t<decltype(src)>>;
-            if (move)
-                hipLaunchKernelGGL((k_move<C, OUT, IN>), dim3((unsigned)(n >> a.nb)), dim3(256), 0, ctx->stream, dst,
-                                   src, n, a, f, usep);
+            if (move) {
+                // (2^22 workgroups a row of the grid: 2^32 threads in one row are refused)
+                const uint64_t tiles = n >> a.nb, row = std::min<uint64_t>(tiles, 1ull << 22);
+                hipLaunchKernelGGL((k_move<C, OUT, IN>), dim3((unsigned)row, (unsigned)(tiles / row)), dim3(256), 0,
+                                   ctx->stream, dst, src, n, a, f, usep);
+            }
             else
                 hipLaunchKernelGGL((k_put<C, OUT, IN>), dim3(grid_for((n + per - 1) / per)), dim3(256), 0,
                                    ctx->stream, dst, src, n, f, usep);
