@@ -239,8 +239,8 @@ def run_c4(prec, circuits, n_seq, steps):
 # Sources each counter summary's kernels are compiled from (the phase programs
 # they apply come from gates.hip).  A summary records their fingerprint; a figure
 # is read from it only while the sources still match.
-FFT_SOURCES = ["fft.hip", "fft_bfly.h", "fft_stages.h", "fft_pass.h", "fft_row.hip", "fft_row.h", "fft_fused.hip", "fft_fused.h", "fft_radix16.h", "diag_fast.h", "cvdv_internal.h", "gates.hip"]
-BATCH_SOURCES = ["batch.hip", "fft_bfly.h", "diag_fast.h", "cvdv_internal.h", "gates.hip"]
+FFT_SOURCES = ["fft.hip", "fft_bfly.h", "fft_stages.h", "fft_pass.h", "fft_row.hip", "fft_row.h", "fft_fused.hip", "fft_fused.h", "fft_radix16.h", "fft_chain.hip", "diag_fast.h", "phase_eval.h", "cvdv_internal.h", "gates.hip"]
+BATCH_SOURCES = ["batch.hip", "fft_bfly.h", "diag_fast.h", "phase_eval.h", "cvdv_internal.h", "gates.hip"]
 
 
 def source_fingerprint(names):
@@ -1079,8 +1079,10 @@ def pmc_traffic(kind):
 # FFT pass kinds of the profile (cvdvProfileRead) -> kernel name and the register
 # transforms one launch performs (a fused pass completes one transform and starts
 # the next: one transform's worth; a lone half: half of one; a row pass, which reads and
-# writes the state once for all the transforms that it chains: counted as one)
-FFT_KINDS = {"fft_fused": ("k_fft_fused", 1.0), "fft_row": ("k_fft_row", 1.0),
+# writes the state once for all the transforms that it chains: counted as one).  "fft_row" counts
+# passes of whole contiguous rows whichever kernel runs them: k_fft_row for this circuit's rows
+# of 2^14 points, a chain or the tile kernel at other sizes and for programs that it does not take.
+FFT_KINDS = {"fft_fused": ("k_fft_fused", 1.0), "fft_row": ("whole-row passes (k_fft_row)", 1.0),
              "fft_half": ("k_fft_tile (four-step half)", 0.5)}
 
 
