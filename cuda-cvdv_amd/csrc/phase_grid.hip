@@ -78,6 +78,17 @@ static void dgemm_tn(CVDVContext* ctx, int m, int n, int k, double alpha, const 
                "rocblas_dgemm_strided_batched");
 }
 
+// The same in complex arithmetic, C = A^T B.
+static void zgemm_tn(CVDVContext* ctx, int m, int n, int k, const double2* A, uint64_t strideA, const double2* B,
+                     double2* C, int ldc, uint64_t strideC, int batch) {
+    const rocblas_double_complex one{1.0, 0.0}, zero{0.0, 0.0};
+    blas_check(rocblas_zgemm_strided_batched(blas(ctx), rocblas_operation_transpose, rocblas_operation_none, m, n, k,
+                                             &one, (const rocblas_double_complex*)A, k, (rocblas_stride)strideA,
+                                             (const rocblas_double_complex*)B, k, 0, &zero,
+                                             (rocblas_double_complex*)C, ldc, (rocblas_stride)strideC, batch),
+               "rocblas_zgemm_strided_batched");
+}
+
 // ---------------------------------------------------------------- kernels
 // X[s][j]: slices of register r in the canonical layout (field at sh), FP64.
 template <typename C>
@@ -281,6 +292,27 @@ __global__ void k_grid_husimi_E(double2* __restrict__ E, const double* __restric
     }
 }
 
+// The operands of the complex form: B[s][q][j] = X[s][j] e^{-(x_j-q)^2/2}, E[p][j] = e^{-i p x_j}.
+__global__ void k_grid_husimi_zB(double2* __restrict__ B, const double2* __restrict__ X, uint64_t S, int n,
+                                 const double* __restrict__ qs, int nqc, double dx) {
+    const uint64_t N = 1ull << n, tot = S * (uint64_t)nqc * N;
+    for (uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; e < tot;
+         e += (uint64_t)gridDim.x * blockDim.x) {
+        const uint64_t j = e & (N - 1), sq = e >> n, q = sq % nqc, s = sq / nqc;
+        const double a = ((double)j - 0.5 * (double)(N - 1)) * dx - qs[q], w = exp(-0.5 * a * a);
+        const double2 u = X[s * N + j];
+        B[e] = make_double2(u.x * w, u.y * w);
+    }
+}
+__global__ void k_grid_husimi_zE(double2* __restrict__ E, const double* __restrict__ ps, int np, int n, double dx) {
+    const uint64_t N = 1ull << n, tot = (uint64_t)np << n;
+    for (uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; e < tot;
+         e += (uint64_t)gridDim.x * blockDim.x) {
+        const double m = (double)(2 * (int64_t)(e & (N - 1)) - (int64_t)N + 1);
+        E[e] = unit_rev(cvdv_frac(cvdv_frac(-dx * ps[e >> n] / (4.0 * PI)) * m), 0.0);
+    }
+}
+
 // out[(s,) p][q] = scale * (|H_s|^2, or summed over s in slice order).
 __global__ void k_grid_abs2(double* __restrict__ out, const double2* __restrict__ H, uint64_t S, uint64_t per,
                             int perSlice, double scale) {
@@ -434,6 +466,15 @@ static void get_wigner_grid(CVDVContext* ctx, int r, const double* xs, int nx, c
     copy_to_host(ctx->stream, out, dout, nZ * sizeof(double));
 }
 
+// Many slices of a short register on a large window: the output of the product is its time, and
+// the library's real kernels (tiles of depth 32) write it more slowly than its complex ones.  Us,
+// real against complex, 256 x 256 points: 2^4 points 912 / 798 under 1024 slices, 269 / 274 under 256;
+// 2^5 1028 / 918; 2^6 1154 / 1145; 2^7 1481 / 1650.  8 x 8: 2^4 points 72 / 83 under 1024 slices; 64 x 64:
+// 2^3 309 / 310, 2^2 359 / 331; 32 x 32: 2^3 355 / 329.
+static bool husimi_grid_complex(int n, uint64_t S, uint64_t points) {
+    return n <= 5 && S >= 512 && points >= (n <= 3 ? 1u << 10 : 1u << 14);
+}
+
 static void get_husimi_grid(CVDVContext* ctx, int r, const double* qs, int nq, const double* ps, int np,
                             int perSlice, double* out) {
     const int n = ctx->nq[r], N = 1 << n, half = N > 1 ? N / 2 : 1;
@@ -445,7 +486,8 @@ static void get_husimi_grid(CVDVContext* ctx, int r, const double* qs, int nq, c
     for (int i = 0; i < nq; ++i) far = std::max(far, std::fabs(qs[i]));
     const double outside = 0.5 * (double)(N - 1) - (far + 38.7) / dx;  // points j below this
     const int j0 = outside >= 16.0 ? std::min((int)std::floor(outside), half - 1) & ~15 : 0;
-    const int nj = half - j0, K = 2 * nj;
+    const bool cplx = husimi_grid_complex(n, S, (uint64_t)np * nq);
+    const int nj = cplx ? N : half - j0, K = cplx ? N : 2 * nj;
     int nqc = nq;
     while (nqc > 1 && (uint64_t)nqc * S * K > GRID_CHUNK) nqc = (nqc + 1) / 2;
     const uint64_t nB = (uint64_t)nqc * S * K, nE = (uint64_t)np * nj, nH = S * (uint64_t)np * nq;
@@ -463,7 +505,10 @@ static void get_husimi_grid(CVDVContext* ctx, int r, const double* qs, int nq, c
     double* dout = g.take<double>(nOut);
     grid_slices(ctx, r, X);
     HIPCHK(hipMemcpyAsync(dqs, up.data(), up.size() * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-    hipLaunchKernelGGL(k_grid_husimi_E, dim3(grid_for(nE)), dim3(256), 0, ctx->stream, E, dps, np, n, dx, j0, nj);
+    if (cplx)
+        hipLaunchKernelGGL(k_grid_husimi_zE, dim3(grid_for(nE)), dim3(256), 0, ctx->stream, E, dps, np, n, dx);
+    else
+        hipLaunchKernelGGL(k_grid_husimi_E, dim3(grid_for(nE)), dim3(256), 0, ctx->stream, E, dps, np, n, dx, j0, nj);
     HIPCHK(hipGetLastError());
     if (j0 > 0) {
         hipLaunchKernelGGL(k_grid_outside, dim3((unsigned)S), dim3(256), 0, ctx->stream, nil, X, n, j0);
@@ -471,6 +516,14 @@ static void get_husimi_grid(CVDVContext* ctx, int r, const double* qs, int nq, c
     }
     for (int q0 = 0; q0 < nq; q0 += nqc) {
         const int c = nq - q0 < nqc ? nq - q0 : nqc;
+        if (cplx) {
+            hipLaunchKernelGGL(k_grid_husimi_zB, dim3(grid_for((uint64_t)c * S * N)), dim3(256), 0, ctx->stream, B, X,
+                               S, n, dqs + q0, c, dx);
+            HIPCHK(hipGetLastError());
+            // H_s[p][q0 + q] = sum_j E[p][j] B[s][q][j]
+            zgemm_tn(ctx, c, np, N, B, (uint64_t)c * N, E, H + q0, nq, (uint64_t)np * nq, (int)S);
+            continue;
+        }
         hipLaunchKernelGGL(k_grid_husimi_B, dim3(grid_for((uint64_t)c * S * nj)), dim3(256), 0, ctx->stream, B, X, S,
                            n, dqs + q0, c, dx, j0, nj, j0 > 0 ? nil : nullptr);
         HIPCHK(hipGetLastError());
