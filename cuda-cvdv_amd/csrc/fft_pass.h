@@ -69,11 +69,18 @@ struct PreLds {
 // The generic terms over a one-row tile (only the transformed field
 // [fs, fs + fn) varies inside it): when every term is affine in that field's
 // coordinate m, their sum is a·m + b (mod 1) with per-tile a, b, and one FP64
-// fma per element replaces the per-term evaluation.  a is reduced mod 1 (m is
-// an integer), so a·m stays below 2^(fn-1) and keeps ~2^-40 absolute accuracy.
+// product per element replaces the per-term evaluation.  a is reduced mod 1 (m is
+// an integer); al is what its rounding left of a bilinear term's slope, and a·m,
+// up to 2^(fn-1) revolutions, is reduced before it is rounded.
 struct GenFold {
-    double a, b;
+    double a, al, b;
     int ok;
+    __device__ __forceinline__ double turn(double m) const { return fma(al, m, fma(a, m, -rint(a * m))); }
+    __device__ __forceinline__ void slope(double c, double m) {
+        const double p = c * m;
+        a += cvdv_frac(p);
+        al += fma(c, m, -p);
+    }
 };
 
 __device__ __forceinline__ bool field_overlaps(int sh, int nb, int fs, int fn) {
@@ -82,7 +89,7 @@ __device__ __forceinline__ bool field_overlaps(int sh, int nb, int fs, int fn) {
 
 __device__ __forceinline__ GenFold fold_generic(const DiagTerm* gen, int ngen, double genrev, uint64_t g0, int fs,
                                                 int fn) {
-    GenFold f{0.0, genrev, 1};
+    GenFold f{0.0, 0.0, genrev, 1};
     for (int i = 0; i < ngen; ++i) {
         const DiagTerm& T = gen[i];
         if (T.ctrl >= 0 && T.ctrl >= fs && T.ctrl < fs + fn) f.ok = 0;
@@ -94,9 +101,9 @@ __device__ __forceinline__ GenFold fold_generic(const DiagTerm* gen, int ngen, d
                 (in1 && in2))
                 f.ok = 0;
             else if (in1)
-                f.a += cvdv_frac(sg * T.c1 * diag_field_m(g0, T.sh2, T.nb2));
+                f.slope(sg * T.c1, diag_field_m(g0, T.sh2, T.nb2));
             else if (in2)
-                f.a += cvdv_frac(sg * T.c1 * diag_field_m(g0, T.sh1, T.nb1));
+                f.slope(sg * T.c1, diag_field_m(g0, T.sh1, T.nb1));
             else
                 f.b += cvdv_frac(sg * diag_term_rev(T, g0));
         } else if (T.kind == DT_POLY || T.kind == DT_LINF) {
@@ -402,7 +409,7 @@ __device__ __forceinline__ void stage0_pre(C* x, const FftPass& d, uint64_t inBa
         } else if (pre.ngen > 0) {
             asm volatile("" : "+v"(tt));
             // one-row tiles: the terms are affine in the row coordinate
-            GenFold gf{0.0, 0.0, 0};
+            GenFold gf{0.0, 0.0, 0.0, 0};
             if (LGC == 0 && d.lgHb == 0) gf = fold_generic(P.gen, pre.ngen, pre.genrev, inBase, d.lgInR, LGM);
             if (gf.ok) {
                 using R = decltype(C{}.x);
@@ -413,19 +420,19 @@ __device__ __forceinline__ void stage0_pre(C* x, const FftPass& d, uint64_t inBa
                 if (nt >= 64) {
                     // full waves: lane i evaluates step i, the others read it
                     const int li = (int)__builtin_amdgcn_mbcnt_lo(~0u, 0u) & (RP - 1);
-                    const C mine = unit_rev_fast(cvdv_frac(gf.a * (double)(2 * (li << lgMq))), R(0));
+                    const C mine = unit_rev_fast(cvdv_frac(gf.turn((double)(2 * (li << lgMq)))), R(0));
 #pragma unroll
                     for (int i = 1; i < RP; ++i) st[i] = lane_value(mine, i);
                 } else {
 #pragma unroll
                     for (int i = 1; i < RP; ++i)
-                        st[i] = unit_rev_fast(cvdv_frac(gf.a * (double)(2 * (i << lgMq))), R(0));
+                        st[i] = unit_rev_fast(cvdv_frac(gf.turn((double)(2 * (i << lgMq)))), R(0));
                 }
 #pragma unroll
                 for (int k = 0; k < NB; ++k) {
                     const BflyPos p = bfly_pos<RP, LGM, E>(tt, k, nt, LGC);
                     const double m0 = (double)(2 * p.q + 1 - (1 << LGM));
-                    const C e0 = unit_rev_fast(cvdv_frac(fma(gf.a, m0, gf.b)), R(0));
+                    const C e0 = unit_rev_fast(cvdv_frac(gf.turn(m0) + gf.b), R(0));
                     x[k * RP] = cmul(x[k * RP], e0);
 #pragma unroll
                     for (int i = 1; i < RP; ++i) x[k * RP + i] = cmul(x[k * RP + i], cmul(e0, st[i]));

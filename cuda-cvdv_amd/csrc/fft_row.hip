@@ -195,14 +195,14 @@ k_fft_row(RowArgs a, typename CT<R>::type* data, const typename CT<R>::type* __r
                 // shares (lane i evaluates step i)
                 const GenFold gf = fold_generic(st.pre.gen, ngen, st.pre.genrev, base, 0, LGM);
                 const int li = (int)__builtin_amdgcn_mbcnt_lo(~0u, 0u) & (E / 4 - 1);
-                const C mine = unit_rev_fast(cvdv_frac(gf.a * (double)(2 * li * (4 * NT))), R(0));
+                const C mine = unit_rev_fast(cvdv_frac(gf.turn((double)(2 * li * (4 * NT)))), R(0));
                 C by[E / 4];
 #pragma unroll
                 for (int i = 1; i < E / 4; ++i) by[i] = lane_value(mine, i);
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
                     const C e0 =
-                        unit_rev_fast(cvdv_frac(fma(gf.a, (double)(2 * (ti + k * NT) + 1 - M), gf.b)), R(0));
+                        unit_rev_fast(cvdv_frac(gf.turn((double)(2 * (ti + k * NT) + 1 - M)) + gf.b), R(0));
                     row_factor(x[k], e0);
 #pragma unroll
                     for (int i = 1; i < E / 4; ++i) row_factor(x[k + 4 * i], cmul(e0, by[i]));

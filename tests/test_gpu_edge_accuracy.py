@@ -101,3 +101,31 @@ def test_edge(gate, n):
     err = np.linalg.norm((h.getState().reshape(psi.shape) - ref(psi.astype(CL))).astype(np.complex128))
     print(f"[edge accuracy] {gate} {regs}: {err:.3e}", flush=True)
     assert err <= 2e-15
+
+
+@pytest.mark.parametrize("regs", [[12, 12], [11, 12], [10, 13]], ids=str)
+def test_rows_under_a_bilinear_phase(regs):
+    """A transform of contiguous rows above 2^22 amplitudes with e^{i t q1 q2} pending: the term is
+    affine in the row, its slope up to a quarter revolution a point.  Rows of the edge and the
+    middle by themselves; relative to each row.  (Unequal sizes round the coefficient itself, by
+    2^-53 of up to 2^8 revolutions, so they are compared with the coefficient that is held.)"""
+    import torch
+    from hipcvdv import HipCvdv
+
+    a, n = regs
+    t = 0.7
+    g = torch.Generator(device="cuda").manual_seed(9)
+    psi = torch.view_as_complex(torch.randn(1 << a, 1 << n, 2, dtype=torch.float64, device="cuda", generator=g))
+    psi /= torch.linalg.vector_norm(psi)
+    h = HipCvdv(regs)
+    h.initFromArray(psi.reshape(-1))
+    h.q1q2(0, 1, t)
+    h.ftQ2P(1)
+    rows = [0, 1, (1 << a - 1) - 1, (1 << a) - 2, (1 << a) - 1]
+    got = h.getStateTensor().reshape(psi.shape)[rows].cpu().numpy()
+    src = psi[rows].cpu().numpy().astype(CL)
+    c = t / (4.0 * 2 ** n) if a == n else t * h.grid_steps[0] * h.grid_steps[1] / (8.0 * math.pi)
+    exp = _ft(src * _turn(L(c) * np.outer(_m(a)[rows], _m(n))), 1, False)
+    err = np.linalg.norm((got - exp).astype(complex), axis=1) / np.linalg.norm(exp.astype(complex), axis=1)
+    print(f"[edge accuracy] rows {regs}: {err}", flush=True)
+    assert np.max(err) <= 1e-15
