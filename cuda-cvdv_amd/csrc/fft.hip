@@ -1089,6 +1089,7 @@ static void settle_one(CVDVContext* ctx, FtDefer& rec) {
 }
 
 void fft_settle(CVDVContext* ctx, bool mayAllocate) {
+    chain_flush(ctx);  // (may leave a half pending)
     if (!ctx->defer.any()) return;
     if (!mayAllocate && !ctx->buf[1 - ctx->cur])
         for (const FtDefer& d : ctx->defer.f)

@@ -707,6 +707,9 @@ static DiagTerm bilin_term(CVDVContext* ctx, int r1, int r2, double coeff, int c
 static void ft_turned(CVDVContext* ctx, int reg, bool inverse, int ctrl) {
     const int nb = ctx->nq[reg];
     if (nb == 0) return;  // N = 1: the transform is the identity
+    // another register's collected transforms run first: one of them by itself may leave a half
+    // pending on a field that this one's phases read
+    if (!ctx->rec && ctx->chain.n > 0 && ctx->chain.sh != ctx->pshift[reg]) chain_flush(ctx);
     const uint64_t N = (uint64_t)1 << nb;
     const double sgn = inverse ? -1.0 : 1.0;
     // Centred DFT: F[k,j] = N^-1/2 exp(-2 pi i m_j m_k / (4N)) =
@@ -880,6 +883,7 @@ static void ft_cparity(CVDVContext* ctx, int tgt, bool inverse, int creg, int cq
         cparity(ctx, tgt, creg, cq);
         return;
     }
+    if (ctx->chain.n > 0 && ctx->chain.sh != ctx->pshift[tgt]) chain_flush(ctx);
     fft_settle_bits(ctx, 1ull << ctrl);
     // logical control bit = NOT physical bit in a reflected register
     ft_turned(ctx, tgt, inverse != (ctx->refl[creg] != 0), ctrl);
