@@ -7,11 +7,15 @@
 // e^{-2 pi i E / 32} as float constants.  Nearest roundings of cos and sin leave |w|^2 - 1
 // of up to 6e-8, which an inner product of 21 fixed constants per stage would turn into a
 // drift of the norm; each pair below is within an ulp of the exact value, and the uses of
-// one stage sum to 4e-8 over 32 elements.
-template <typename R, int E> struct W32;
-template <int E> struct W32<float, E> {
+// one stage sum to 4e-8 over 32 elements.  A localised state reaches a stage through one of
+// its inputs alone, so the constants that one input meets have to balance too: between the two
+// steps of 32 points (INNER) W^15 is the pair of the other side, since the products of input 3,
+// W^{3 m}, had summed to 8e-8 (now -3e-8, as those of input 1; input 2 -1e-8).
+template <typename R, int E, bool INNER> struct W32;
+template <int E, bool INNER> struct W32<float, E, INNER> {
     static constexpr int q = (E >> 3) & 3, r = E & 7;
-    static constexpr float c1 = (E & 31) == 1 ? 0.9807852506637573f : 0.9807853102684021f;
+    static constexpr float c1 =
+        (E & 31) == 1 || (INNER && (E & 31) == 15) ? 0.9807852506637573f : 0.9807853102684021f;
     static constexpr float s1 = 0.19509032368659973f;
     static constexpr float c2 = (E & 31) == 6 || (E & 31) == 14 ? 0.9238795042037964f : 0.9238795638084412f;
     static constexpr float s2 = 0.3826834261417389f;
@@ -20,7 +24,7 @@ template <int E> struct W32<float, E> {
     static constexpr float s = r == 1 ? s1 : r == 2 ? s2 : r == 3 ? s3 : r == 5 ? c3 : r == 6 ? c2 : c1;
 };
 
-template <int E> struct W32<double, E> {
+template <int E, bool INNER> struct W32<double, E, INNER> {
     static constexpr int q = (E >> 3) & 3, r = E & 7;
     static constexpr double c1 = 0.98078528040323044913, s1 = 0.19509032201612826785;
     static constexpr double c2 = 0.92387953251128675613, s2 = 0.38268343236508977173;
@@ -29,9 +33,9 @@ template <int E> struct W32<double, E> {
     static constexpr double s = r == 1 ? s1 : r == 2 ? s2 : r == 3 ? s3 : r == 5 ? c3 : r == 6 ? c2 : c1;
 };
 
-template <int E, typename C>
+template <int E, bool INNER = false, typename C>
 __device__ __forceinline__ C mul_w32(C a) {
-    using W = W32<decltype(C{}.x), E>;
+    using W = W32<decltype(C{}.x), E, INNER>;
     C t = a;
     if constexpr (W::r == 4) {
         t.x = mul_rsqrt2(a.x + a.y);

@@ -39,7 +39,7 @@ __device__ __forceinline__ void dft8_at(C* x) {
 }
 template <int K, int M2>
 __device__ __forceinline__ void dft32_inner(float2* x) {
-    x[K + 4 * M2] = mul_w32<K * M2>(x[K + 4 * M2]);
+    x[K + 4 * M2] = mul_w32<K * M2, true>(x[K + 4 * M2]);
     if constexpr (M2 < 7) dft32_inner<K, M2 + 1>(x);
     else if constexpr (K < 3) dft32_inner<K + 1, 1>(x);
 }
